@@ -55,6 +55,19 @@ int ts_contract2(const uint8_t* lhs, int32_t lhs_rank, const int32_t* lhs_wires,
                  uint8_t* out, int32_t out_rank, const int32_t* out_wires, int32_t mode,
                  ts_stream stream);
 
+/* The same contraction with scratch memory for operands whose wire order is permuted first
+ * (a summed wire that is not innermost, kept wires out of the out order): `bytes` receives
+ * what a 16-byte aligned call of these wires can use (0: none), and ts_contract2_into takes
+ * that much device memory, 16-byte aligned, for the launches it makes on `stream`.  With less
+ * (or NULL, 0) it runs like ts_contract2, which has none. */
+int ts_contract2_scratch(int32_t lhs_rank, const int32_t* lhs_wires, int32_t rhs_rank,
+                         const int32_t* rhs_wires, int32_t out_rank, const int32_t* out_wires,
+                         int64_t* bytes);
+int ts_contract2_into(const uint8_t* lhs, int32_t lhs_rank, const int32_t* lhs_wires,
+                      const uint8_t* rhs, int32_t rhs_rank, const int32_t* rhs_wires,
+                      uint8_t* out, int32_t out_rank, const int32_t* out_wires, int32_t mode,
+                      uint8_t* scratch, int64_t scratch_bytes, ts_stream stream);
+
 /* FinRel._rewire (fin_rel.py:379-393) and rewire_array (_utils/misc.py:104-123):
  * out axes are input ports, possibly repeated (diagonal embedding) or absent
  * (existential sum).  Pure permutations run the permute path. */

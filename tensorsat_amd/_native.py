@@ -22,6 +22,7 @@ TS_EUNSUPPORTED = -3
 TS_EOVERFLOW = -4
 TS_EHIP = -5
 BATCH_LDS_MAX = 65536
+SCRATCH_MIN_BITS = 12  # contractions without a tensor of this rank never take scratch memory
 BATCH_SEGMENTS = 8  # queue counters per dispatch (TS_BATCH_SEGMENTS)
 BATCH_COUNTER_STRIDE = 64  # int32s between queue counters (TS_BATCH_COUNTER_STRIDE)
 BATCH_COUNTER_INTS = BATCH_SEGMENTS * BATCH_COUNTER_STRIDE
@@ -32,7 +33,7 @@ MODES = {"GT0": MODE_GT0, "MOD256": MODE_MOD256}
 
 # Every symbol declared in include/tensorsat_amd.h.
 EXPORTS = (
-    "ts_init", "ts_version", "ts_contract2", "ts_rewire", "ts_spider", "ts_union", "ts_stack",
+    "ts_init", "ts_version", "ts_contract2", "ts_contract2_scratch", "ts_contract2_into", "ts_rewire", "ts_spider", "ts_union", "ts_stack",
     "ts_select", "ts_as_scalar", "ts_diagonal", "ts_count_contract2", "ts_bytes_to_u64",
     "ts_program_run", "ts_program_count", "ts_batch_run", "ts_batch_max_workgroups",
     "ts_batch_compact", "ts_batch_count", "ts_batch_max_workgroups_lds", "ts_gnn_gemm", "ts_gnn_segsum", "ts_gnn_relu_back",
@@ -70,6 +71,8 @@ def load() -> ctypes.CDLL:
         L.ts_init.argtypes = [ctypes.c_int]
         L.ts_version.restype = ctypes.c_char_p
         L.ts_contract2.argtypes = [vp, i32, P(i32), vp, i32, P(i32), vp, i32, P(i32), i32, vp]
+        L.ts_contract2_scratch.argtypes = [i32, P(i32), i32, P(i32), i32, P(i32), P(i64)]
+        L.ts_contract2_into.argtypes = [vp, i32, P(i32), vp, i32, P(i32), vp, i32, P(i32), i32, vp, i64, vp]
         L.ts_count_contract2.argtypes = [vp, i32, P(i32), vp, i32, P(i32), vp, i32, P(i32), vp, vp]
         L.ts_rewire.argtypes = [vp, i32, vp, i32, P(i32), i32, vp]
         L.ts_diagonal.argtypes = [vp, i32, P(i32), vp, i32, vp]

@@ -131,6 +131,115 @@ __global__ __launch_bounds__(WG) void k_step_dot(const uint8_t* __restrict__ lhs
   dot_block(st, L, lhs, rhs, out, blockIdx.x, mode, part);
 }
 
+// Bit 7 of each byte set iff that byte of x is nonzero (the other bits clear).
+__device__ __forceinline__ uint32_t nonzero_bytes(uint32_t x) {
+  return (((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x) & 0x80808080u;
+}
+
+// Products summed outside: each operand's kept bits are in out order from its lowest bit, its
+// summed bits anywhere above the 2^4-output chunks (at most 7 of them: a count of at most
+// 128, so both epilogues are "any term set").  A lane computes 16 consecutive outputs: for
+// every term it loads one chunk of each operand (2^HL / 2^HR bytes, HL / HR = the low four out
+// bits that operand holds), spreads it over the 16 bytes with v_perm, and ORs the AND of
+// both.  Lanes are consecutive groups of outputs, so the chunks of a wave are whole runs.
+// Bound by HBM: operands and result once each, up to four terms' loads in flight per lane.
+struct OuterArgs {
+  int32_t out_rank, nc;
+  uint32_t sel[2][4];             // v_perm selectors: output dword q from an operand's chunk
+  uint32_t bit[2][TS_MAX_BITS];   // operand offset of out bit j (0: not held)
+  uint32_t term[2][8];            // operand offset of summed bit j
+};
+
+template <int H>
+struct Chunk {
+  uint32_t w[H < 4 ? 2 : 4];
+};
+
+template <int H>
+__device__ __forceinline__ Chunk<H> chunk_load(const uint8_t* p) {
+  Chunk<H> c;
+  if constexpr (H == 4) {
+    const uint4 v = *reinterpret_cast<const uint4*>(p);
+    c.w[0] = v.x;
+    c.w[1] = v.y;
+    c.w[2] = v.z;
+    c.w[3] = v.w;
+  } else if constexpr (H == 3) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    c.w[0] = v.x;
+    c.w[1] = v.y;
+  } else {
+    c.w[1] = 0;
+    if constexpr (H == 2) c.w[0] = *reinterpret_cast<const uint32_t*>(p);
+    else if constexpr (H == 1) c.w[0] = *reinterpret_cast<const uint16_t*>(p);
+    else c.w[0] = *p;
+  }
+  return c;
+}
+
+// Output dword q (outputs 4q .. 4q + 3) of a chunk.
+template <int H>
+__device__ __forceinline__ uint32_t chunk_dword(const Chunk<H>& c, int q, const uint32_t (&sel)[4]) {
+  if constexpr (H == 4) return c.w[q];
+  else return __builtin_amdgcn_perm(c.w[1], c.w[0], sel[q]);
+}
+
+template <int HL, int HR, int NT>
+__device__ __forceinline__ void outer_tiles(const uint8_t* __restrict__ lhs, const uint8_t* __restrict__ rhs,
+                                            uint8_t* __restrict__ out, const OuterArgs& a) {
+  const int tid = threadIdx.x;
+  uint32_t lane_l = 0, lane_r = 0;  // out bits 4..11 from the thread
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if ((tid >> i) & 1) {
+      lane_l += a.bit[0][4 + i];
+      lane_r += a.bit[1][4 + i];
+    }
+  const uint32_t ntiles = 1u << (a.out_rank - 12), nterm = 1u << a.nc;
+  for (uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    uint32_t bl = 0, br = 0;
+    for (int j = 12; j < a.out_rank; ++j)
+      if ((t >> (j - 12)) & 1u) {
+        bl += a.bit[0][j];
+        br += a.bit[1][j];
+      }
+    const uint8_t* pl = lhs + bl + lane_l;
+    const uint8_t* pr = rhs + br + lane_r;
+    uint32_t res[4] = {0, 0, 0, 0};
+    for (uint32_t c0 = 0; c0 < nterm; c0 += NT) {
+      Chunk<HL> x[NT];
+      Chunk<HR> y[NT];
+#pragma unroll
+      for (int u = 0; u < NT; ++u) {
+        uint32_t tl = 0, tr = 0;
+        for (int j = 0; j < a.nc; ++j)
+          if (((c0 + u) >> j) & 1u) {
+            tl += a.term[0][j];
+            tr += a.term[1][j];
+          }
+        x[u] = chunk_load<HL>(pl + tl);
+        y[u] = chunk_load<HR>(pr + tr);
+      }
+#pragma unroll
+      for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) res[q] |= chunk_dword<HL>(x[u], q, a.sel[0]) & chunk_dword<HR>(y[u], q, a.sel[1]);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) res[q] = nonzero_bytes(res[q]) >> 7;
+    const uint64_t o = ((uint64_t)t << 12) | ((uint32_t)tid << 4);
+    *reinterpret_cast<uint4*>(out + o) = make_uint4(res[0], res[1], res[2], res[3]);
+  }
+}
+
+template <int HL, int HR>
+__global__ __launch_bounds__(WG) void k_step_outer(const uint8_t* __restrict__ lhs, const uint8_t* __restrict__ rhs,
+                                                   uint8_t* __restrict__ out, OuterArgs a) {
+  if (a.nc == 0) outer_tiles<HL, HR, 1>(lhs, rhs, out, a);
+  else if (a.nc == 1) outer_tiles<HL, HR, 2>(lhs, rhs, out, a);
+  else outer_tiles<HL, HR, 4>(lhs, rhs, out, a);
+}
+
 // Descriptor structs passed by value are read through the kernel-argument segment
 // (uniform scalar loads, no private copy of their arrays).
 template <class T>
@@ -611,11 +720,6 @@ __global__ __launch_bounds__(WG) void k_zero16(uint4* __restrict__ p, uint64_t n
     p[i] = make_uint4(0, 0, 0, 0);
 }
 
-// Bit 7 of each byte set iff that byte of x is nonzero (the other bits clear).
-__device__ __forceinline__ uint32_t nonzero_bytes(uint32_t x) {
-  return (((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x) & 0x80808080u;
-}
-
 template <int NKB>
 __global__ __launch_bounds__(WG) void k_reduce_w16(const uint8_t* __restrict__ in, uint8_t* __restrict__ out,
                                                    ReduceWideArgs a) {
@@ -892,6 +996,237 @@ int launch_step_u64(const uint64_t* lhs, const uint64_t* rhs, uint64_t* out, con
   return hip_rc(hipGetLastError());
 }
 
+// Bit permutation out[o] = in[pi(o)] of a 2^r-byte tensor: out bit q comes from in bit pi[q].
+int launch_permute(const uint8_t* in, uint8_t* out, const int* pi, int r, hipStream_t s) {
+  const int b = std::min(PB, r);
+  PermArgs pa;
+  std::memset(&pa, 0, sizeof(pa));
+  int Sout[2 * PB], Sin[2 * PB];
+  for (int q = 0; q < r; ++q) {
+    if (q < b || pi[q] < b) {
+      Sout[pa.s] = q;
+      Sin[pa.s++] = q;
+    } else {
+      pa.rest_out[pa.nr] = (uint8_t)q;
+      pa.rest_in[pa.nr++] = (uint8_t)pi[q];
+    }
+  }
+  std::sort(Sin, Sin + pa.s, [&](int x, int y) { return pi[x] < pi[y]; });
+  for (int k = 0; k < pa.s; ++k) {
+    pa.load_in[k] = (uint8_t)pi[Sin[k]];
+    pa.load_lds[k] = (uint8_t)(std::find(Sout, Sout + pa.s, Sin[k]) - Sout);
+    pa.store_out[k] = (uint8_t)Sout[k];
+  }
+  const uint64_t ntiles = 1ull << pa.nr;
+  const int grid = (int)std::min<uint64_t>(ntiles, 65536);
+  const bool aligned = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+  if (pa.s >= 4 && aligned)
+    hipLaunchKernelGGL(k_permute_lds16, dim3(grid), dim3(WG), 0, s, in, out, pa);
+  else
+    hipLaunchKernelGGL(k_permute_lds, dim3(grid), dim3(WG), 0, s, in, out, pa);
+  return hip_rc(hipGetLastError());
+}
+
+// ---- pairwise contractions with arbitrary wire orders ----------------------------------
+//
+// The step engine is fast on one family of layouts: summed bits innermost in both operands,
+// or short rows next to the out order.  A contraction as a program writes it has its wires
+// in any order, and a byte gather per term then touches a whole line for each byte it uses.
+// Such an operand is first permuted (launch_permute: both sides coalesced) into scratch
+// memory of the caller, in the layout its kernel reads best.
+enum : int { PLAN_NONE, PLAN_OUTER, PLAN_DENSE, PLAN_INNER };
+struct ContractPlan {
+  int kind;
+  bool move_l, move_r;                        // operand is permuted first
+  int pi_l[TS_MAX_BITS], pi_r[TS_MAX_BITS];   // its permutation (new bit -> old bit)
+  int64_t at_r, bytes;                        // scratch: rhs copy's offset, all bytes
+  ts_step st;                                 // the step on the (permuted) operands
+};
+
+// Kept bits of one operand in out order, at the lowest positions up to the first `run`.
+bool runs_in_order(const ts_step& st, const uint8_t* pos, int run) {
+  int k = 0;
+  for (int j = 0; j < st.out_rank && k < run; ++j)
+    if (pos[j] != TS_NOPOS && pos[j] != k++) return false;
+  return true;
+}
+
+// New layout of one operand: kept bits in out order below (inner = false) or above (inner =
+// true) its summed bits, which follow the record's order.
+void regular_layout(ts_step& st, uint8_t* pos, uint8_t* cpos, bool inner, int* pi) {
+  int n = 0;
+  auto summed = [&]() {
+    for (int j = 0; j < st.sum_rank; ++j) {
+      pi[n] = cpos[j];
+      cpos[j] = (uint8_t)n++;
+    }
+  };
+  if (inner) summed();
+  for (int j = 0; j < st.out_rank; ++j)
+    if (pos[j] != TS_NOPOS) {
+      pi[n] = pos[j];
+      pos[j] = (uint8_t)n++;
+    }
+  if (!inner) summed();
+}
+
+// The rule (every summed wire held by both operands -- a wire summed in one operand only
+// stays with the step engine, MOD256 counts multiply there -- and 16-byte aligned operands):
+//  * 6 or more summed bits, 4 or more bits held by one operand only on each side, 2^DENSE_MIN
+//    or more products: the summed bits are moved innermost and the matrix cores run the
+//    product.  2^13 x 2^13 by 2^13 x 2^13: 602 ms as byte gathers, 0.50 ms so (0.03 ms of it
+//    the permutation); 2^6 x 2^10 by 2^10 x 2^6: 22 -> 13 us;
+//  * at most 7 summed bits (128 terms: both epilogues are "any") and 2^OUT_MIN or more
+//    outputs: k_step_outer, the kept bits of each operand in out order (in runs of 64 bytes;
+//    an operand that has them so is read in place, wherever its summed bits are above).
+//    2^25 and 2^24 entries into 2^26 over one summed bit: 291 -> 50 us.  At 2^20 outputs
+//    16 -> 12 us, at 2^18 the two or three launches lose (9 -> 15 us), hence the line;
+//  * otherwise, 2^TERM_MIN or more products: summed bits innermost for the popcount rows of
+//    the step engine.
+// A step already in a layout of the step engine that reads whole runs keeps it.
+constexpr int OUT_MIN = 20, TERM_MIN = 22, DENSE_MIN = 18;
+
+ContractPlan plan_contract(const ts_step& s0, bool aligned) {
+  ContractPlan p;
+  p.kind = PLAN_NONE;
+  p.move_l = p.move_r = false;
+  p.at_r = p.bytes = 0;
+  p.st = s0;
+  ts_step& st = p.st;
+  const int nc = st.sum_rank;
+  if (!aligned || st.out_rank + nc < DENSE_MIN) return p;
+  for (int j = 0; j < nc; ++j)
+    if (st.c_lpos[j] == TS_NOPOS || st.c_rpos[j] == TS_NOPOS) return p;
+  int nm = 0, nn = 0;
+  for (int j = 0; j < st.out_rank; ++j) {
+    nm += st.o_rpos[j] == TS_NOPOS;
+    nn += st.o_lpos[j] == TS_NOPOS;
+  }
+  const bool kinner = st.flags & TS_STEP_KINNER;
+  const bool dense = nc >= 6 && nm >= 4 && nn >= 4;
+  if (dense) {
+    if (kinner) return p;
+    p.kind = PLAN_DENSE;
+  } else if (nc <= 7 && st.out_rank >= OUT_MIN) {
+    uint32_t ml, mr;
+    auto rows_in_order = [&](const uint8_t* pos) {  // kept bits right above the summed ones
+      int k = nc;
+      for (int j = 0; j < st.out_rank && k < 6; ++j)
+        if (pos[j] != TS_NOPOS && pos[j] != k++) return false;
+      return true;
+    };
+    if (kinner && vec_plan(st, ml, mr) == 4 && rows_in_order(st.o_lpos) && rows_in_order(st.o_rpos)) return p;
+    p.kind = PLAN_OUTER;
+  } else {
+    if (kinner || st.out_rank + nc < TERM_MIN) return p;
+    p.kind = PLAN_INNER;
+  }
+  if (p.kind == PLAN_OUTER) {
+    p.move_l = !runs_in_order(st, st.o_lpos, 6);
+    p.move_r = !runs_in_order(st, st.o_rpos, 6);
+    if (p.move_l) regular_layout(st, st.o_lpos, st.c_lpos, false, p.pi_l);
+    if (p.move_r) regular_layout(st, st.o_rpos, st.c_rpos, false, p.pi_r);
+    st.flags &= ~TS_STEP_KINNER;
+  } else {
+    // The order of the summed bits is free: an operand that has them innermost keeps its
+    // layout (the larger one first; the record's order is the other's).
+    auto lowest = [&](const uint8_t* c) {
+      for (int j = 0; j < nc; ++j)
+        if (c[j] >= nc) return false;
+      return true;
+    };
+    const bool il = lowest(st.c_lpos), ir = lowest(st.c_rpos);
+    if (il || ir) {
+      const bool by_l = il && (!ir || st.lhs_rank >= st.rhs_rank);
+      uint8_t cl[TS_MAX_BITS], cr[TS_MAX_BITS];
+      std::memcpy(cl, st.c_lpos, sizeof(cl));
+      std::memcpy(cr, st.c_rpos, sizeof(cr));
+      for (int j = 0; j < nc; ++j) {
+        const int at = by_l ? cl[j] : cr[j];
+        st.c_lpos[at] = cl[j];
+        st.c_rpos[at] = cr[j];
+      }
+    }
+    auto inner = [&](const uint8_t* c) {
+      for (int j = 0; j < nc; ++j)
+        if (c[j] != j) return false;
+      return true;
+    };
+    p.move_l = !inner(st.c_lpos);
+    p.move_r = !inner(st.c_rpos);
+    if (p.move_l) regular_layout(st, st.o_lpos, st.c_lpos, true, p.pi_l);
+    if (p.move_r) regular_layout(st, st.o_rpos, st.c_rpos, true, p.pi_r);
+    st.flags |= TS_STEP_KINNER;
+  }
+  const int64_t bl = p.move_l ? (1ll << st.lhs_rank) : 0, br = p.move_r ? (1ll << st.rhs_rank) : 0;
+  p.at_r = (bl + 255) & ~255ll;
+  p.bytes = p.at_r + br;
+  return p;
+}
+
+template <int HL>
+int launch_outer_r(const uint8_t* lhs, const uint8_t* rhs, uint8_t* out, const OuterArgs& a, int hr, int grid,
+                   hipStream_t s) {
+  switch (hr) {
+    case 0: hipLaunchKernelGGL((k_step_outer<HL, 0>), dim3(grid), dim3(WG), 0, s, lhs, rhs, out, a); break;
+    case 1: hipLaunchKernelGGL((k_step_outer<HL, 1>), dim3(grid), dim3(WG), 0, s, lhs, rhs, out, a); break;
+    case 2: hipLaunchKernelGGL((k_step_outer<HL, 2>), dim3(grid), dim3(WG), 0, s, lhs, rhs, out, a); break;
+    case 3: hipLaunchKernelGGL((k_step_outer<HL, 3>), dim3(grid), dim3(WG), 0, s, lhs, rhs, out, a); break;
+    default: hipLaunchKernelGGL((k_step_outer<HL, 4>), dim3(grid), dim3(WG), 0, s, lhs, rhs, out, a); break;
+  }
+  return hip_rc(hipGetLastError());
+}
+
+int launch_outer(const uint8_t* lhs, const uint8_t* rhs, uint8_t* out, const ts_step& st, hipStream_t s) {
+  OuterArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.out_rank = st.out_rank;
+  a.nc = st.sum_rank;
+  int h[2] = {0, 0};
+  for (int e = 0; e < 2; ++e) {
+    const uint8_t* pos = e ? st.o_rpos : st.o_lpos;
+    uint32_t mask = 0;
+    for (int j = 0; j < 4; ++j)
+      if (pos[j] != TS_NOPOS) {
+        mask |= 1u << j;
+        ++h[e];
+      }
+    for (int i = 0; i < 16; ++i) {
+      uint32_t idx = 0, b = 0;
+      for (int j = 0; j < 4; ++j)
+        if ((mask >> j) & 1u) idx |= ((uint32_t)(i >> j) & 1u) << b++;
+      a.sel[e][i >> 2] |= (idx & 7u) << (8 * (i & 3));
+    }
+    for (int j = 4; j < st.out_rank; ++j) a.bit[e][j] = pos[j] != TS_NOPOS ? 1u << pos[j] : 0u;
+    const uint8_t* c = e ? st.c_rpos : st.c_lpos;
+    for (int j = 0; j < st.sum_rank; ++j) a.term[e][j] = 1u << c[j];
+  }
+  const int grid = (int)std::min<uint64_t>(1ull << (st.out_rank - 12), 8192);
+  switch (h[0]) {
+    case 0: return launch_outer_r<0>(lhs, rhs, out, a, h[1], grid, s);
+    case 1: return launch_outer_r<1>(lhs, rhs, out, a, h[1], grid, s);
+    case 2: return launch_outer_r<2>(lhs, rhs, out, a, h[1], grid, s);
+    case 3: return launch_outer_r<3>(lhs, rhs, out, a, h[1], grid, s);
+    default: return launch_outer_r<4>(lhs, rhs, out, a, h[1], grid, s);
+  }
+}
+
+int run_contract(const uint8_t* lhs, const uint8_t* rhs, uint8_t* out, const ContractPlan& p, uint8_t* scratch,
+                 int mode, hipStream_t s) {
+  if (p.move_l) {
+    const int rc = launch_permute(lhs, scratch, p.pi_l, p.st.lhs_rank, s);
+    if (rc) return rc;
+    lhs = scratch;
+  }
+  if (p.move_r) {
+    const int rc = launch_permute(rhs, scratch + p.at_r, p.pi_r, p.st.rhs_rank, s);
+    if (rc) return rc;
+    rhs = scratch + p.at_r;
+  }
+  if (p.kind == PLAN_OUTER) return launch_outer(lhs, rhs, out, p.st, s);
+  return launch_step_u8(lhs, rhs, out, p.st, mode, s);
+}
+
 }  // namespace
 
 extern "C" {
@@ -911,11 +1246,34 @@ const char* ts_version(void) { return "tensorsat_amd 0.1.0 (gfx950)"; }
 int ts_contract2(const uint8_t* lhs, int32_t lhs_rank, const int32_t* lhs_wires, const uint8_t* rhs,
                  int32_t rhs_rank, const int32_t* rhs_wires, uint8_t* out, int32_t out_rank,
                  const int32_t* out_wires, int32_t mode, ts_stream stream) {
-  if (!lhs || !rhs || !out || (mode != TS_MODE_GT0 && mode != TS_MODE_MOD256)) return TS_EINVAL;
+  return ts_contract2_into(lhs, lhs_rank, lhs_wires, rhs, rhs_rank, rhs_wires, out, out_rank, out_wires, mode, nullptr,
+                           0, stream);
+}
+
+int ts_contract2_scratch(int32_t lhs_rank, const int32_t* lhs_wires, int32_t rhs_rank, const int32_t* rhs_wires,
+                         int32_t out_rank, const int32_t* out_wires, int64_t* bytes) {
+  if (!bytes) return TS_EINVAL;
   ts_step st;
   int rc = make_step(lhs_rank, lhs_wires, rhs_rank, rhs_wires, out_rank, out_wires, false, st);
   if (rc) return rc;
-  if ((reinterpret_cast<uintptr_t>(lhs) | reinterpret_cast<uintptr_t>(rhs)) & 15) st.flags &= ~TS_STEP_KINNER;
+  *bytes = plan_contract(st, true).bytes;
+  return TS_OK;
+}
+
+int ts_contract2_into(const uint8_t* lhs, int32_t lhs_rank, const int32_t* lhs_wires, const uint8_t* rhs,
+                      int32_t rhs_rank, const int32_t* rhs_wires, uint8_t* out, int32_t out_rank,
+                      const int32_t* out_wires, int32_t mode, uint8_t* scratch, int64_t scratch_bytes,
+                      ts_stream stream) {
+  if (!lhs || !rhs || !out || (mode != TS_MODE_GT0 && mode != TS_MODE_MOD256)) return TS_EINVAL;
+  if (scratch_bytes < 0 || (scratch_bytes > 0 && !scratch)) return TS_EINVAL;
+  ts_step st;
+  int rc = make_step(lhs_rank, lhs_wires, rhs_rank, rhs_wires, out_rank, out_wires, false, st);
+  if (rc) return rc;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(lhs) | reinterpret_cast<uintptr_t>(rhs);
+  const uintptr_t to = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(scratch);
+  if (at & 15) st.flags &= ~TS_STEP_KINNER;
+  const ContractPlan p = plan_contract(st, ((at | to) & 15) == 0);
+  if (p.kind != PLAN_NONE && p.bytes <= scratch_bytes) return run_contract(lhs, rhs, out, p, scratch, mode, S(stream));
   return launch_step_u8(lhs, rhs, out, st, mode, S(stream));
 }
 
@@ -962,37 +1320,9 @@ int ts_rewire(const uint8_t* in, int32_t in_rank, uint8_t* out, int32_t out_rank
     if (a.num_disc == 0) {
       // Bit positions: out bit q is out axis r-1-q; its in bit is r-1-out_port[r-1-q].
       const int r = out_rank;
-      std::vector<int> pi(r);
+      int pi[TS_MAX_BITS];
       for (int q = 0; q < r; ++q) pi[q] = r - 1 - out_ports[r - 1 - q];
-      const int b = std::min(PB, r);
-      std::vector<char> inS(r, 0);
-      for (int q = 0; q < r; ++q)
-        if (q < b || pi[q] < b) inS[q] = 1;
-      std::vector<int> Sout, Sin, rest;
-      for (int q = 0; q < r; ++q) (inS[q] ? Sout : rest).push_back(q);
-      Sin = Sout;
-      std::sort(Sin.begin(), Sin.end(), [&](int x, int y) { return pi[x] < pi[y]; });
-      PermArgs pa;
-      std::memset(&pa, 0, sizeof(pa));
-      pa.s = (int)Sout.size();
-      pa.nr = (int)rest.size();
-      for (int k = 0; k < pa.s; ++k) {
-        pa.load_in[k] = (uint8_t)pi[Sin[k]];
-        pa.load_lds[k] = (uint8_t)(std::find(Sout.begin(), Sout.end(), Sin[k]) - Sout.begin());
-        pa.store_out[k] = (uint8_t)Sout[k];
-      }
-      for (int k = 0; k < pa.nr; ++k) {
-        pa.rest_out[k] = (uint8_t)rest[k];
-        pa.rest_in[k] = (uint8_t)pi[rest[k]];
-      }
-      const uint64_t ntiles = 1ull << pa.nr;
-      const int grid = (int)std::min<uint64_t>(ntiles, 65536);
-      const bool aligned = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-      if (pa.s >= 4 && aligned)
-        hipLaunchKernelGGL(k_permute_lds16, dim3(grid), dim3(WG), 0, s, in, out, pa);
-      else
-        hipLaunchKernelGGL(k_permute_lds, dim3(grid), dim3(WG), 0, s, in, out, pa);
-      return hip_rc(hipGetLastError());
+      return launch_permute(in, out, pi, r, s);
     }
     if (a.num_disc >= 6 && mode == TS_MODE_GT0 && in_rank >= 10 && (reinterpret_cast<uintptr_t>(in) & 15) == 0) {
       // Bits 0..3 in each lane's 16 bytes, bits 4..9 on the lanes.

@@ -361,9 +361,19 @@ class DeviceRel:
         if max(len(bl), len(br), len(bo)) > MAX_DEVICE_BITS:
             raise NotImplementedError("operand exceeds 2^27 device entries")
         res = _empty(1 << len(bo))
-        N.check(N.lib().ts_contract2(
-            N.dptr(lhs._data), len(bl), N.i32arr(bl), N.dptr(rhs._data), len(br), N.i32arr(br),
-            N.dptr(res), len(bo), N.i32arr(bo), N.MODES[DeviceRel._mode], N.stream_ptr()), "ts_contract2")
+        L = N.lib()
+        wl, wr, wo = N.i32arr(bl), N.i32arr(br), N.i32arr(bo)
+        # Operands of large contractions are permuted into scratch memory where their wire
+        # order needs it; it goes back to the allocator on this stream after the launches.
+        need = N.i64(0)
+        if max(len(bl), len(br), len(bo)) >= N.SCRATCH_MIN_BITS:
+            N.check(L.ts_contract2_scratch(len(bl), wl, len(br), wr, len(bo), wo, ctypes.byref(need)),
+                    "ts_contract2_scratch")
+        scratch = _empty(need.value) if need.value else None
+        N.check(L.ts_contract2_into(
+            N.dptr(lhs._data), len(bl), wl, N.dptr(rhs._data), len(br), wr, N.dptr(res), len(bo), wo,
+            N.MODES[DeviceRel._mode], N.dptr(scratch) if need.value else None, need.value, N.stream_ptr()),
+            "ts_contract2")
         box = DeviceRel._new(res, out_shape)
         if len(uniq_out) != len(out_wires):
             box = box._rewire([uniq_out.index(w) for w in out_wires])
