@@ -45,6 +45,11 @@ typedef struct {
 #define TS_STEP_NORHS 2   /* unary step (rewire/reduce): rhs is the constant 1 */
 #define TS_STEP_PACKET 4  /* packet form (tsc_packetize): pad[0] = first lane of this step */
 #define TS_STEP_PEND 8    /* packet form: last record of its packet */
+/* Counting (tsc_count_widths): pad[0] of a step holds the storage of its operands (bits 0-1
+ * lhs, 2-3 rhs: 0 uint64, 1 uint32, 2 uint64 with values below 2^32) and these bits;
+ * 0 means uint64 throughout, checked. */
+#define TS_COUNT_OUT32 16 /* the result is stored as uint32 */
+#define TS_COUNT_EXACT 32 /* no product or sum of this step reaches 2^64 */
 #define TS_PACKET_LANES 64 /* lanes of one packet (one wavefront) */
 #define TS_PACKET_CHUNK 16 /* packets never straddle a boundary of this many records of a job */
 
@@ -149,6 +154,16 @@ int tsc_sat_batch(int32_t num_inst, const int32_t* nvars, const int64_t* clause_
  * step to have at most 6 out bits and no packet flags yet (TSP_EINVAL otherwise, jobs
  * already done stay packetized).  threads <= 0: hardware concurrency. */
 int tsc_packetize(ts_job* jobs, int64_t num_jobs, ts_step* steps, int64_t num_steps, int32_t threads);
+
+/* Storage widths of a counting program (no counterpart in the reference: an execution layout
+ * of this build): a tensor's entries are at most 2^b, b = the summed bits of all steps under
+ * it (plus 8 per leaf if the job has a leaf byte above 1).  Writes pad[0] of every step
+ * (TS_COUNT_*); the tensor at a job's result_off stays uint64, and so does every step of a
+ * job whose operands are not whole tensors written before (pad[0] = 0).  Offsets and arena
+ * sizes stay as they are: a uint32 tensor fills half its room.  threads <= 0: hardware
+ * concurrency. */
+int tsc_count_widths(const ts_job* jobs, int64_t num_jobs, ts_step* steps, int64_t num_steps,
+                     const uint8_t* leaves, int64_t num_leaf_bytes, int32_t threads);
 
 /* Lane form of a packet-form program (no counterpart in the reference: an execution
  * layout of this build): one 16-byte record per lane of every packet, all index math

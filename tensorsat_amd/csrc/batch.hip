@@ -471,10 +471,219 @@ __global__ __launch_bounds__(64) void k_batch_wave(ts_batch b) {
   }
 }
 
-// Counting semiring: the same walk with uint64 arenas (arena_stride is in bytes) and
-// checked arithmetic; each job's scalar result times 2^free_vars is added to its
+// ---- counting semiring ---------------------------------------------------------------
+//
+// The same walk over (+, x) with exact integer counts: an arena element is 8 bytes wide, and
+// a tensor whose record proves its entries below 2^32 (tsc_count_widths: at most 2^b with b
+// the summed bits under it) is stored as uint32 at the start of its room, so a step reads and
+// writes half the bytes.  Records without that proof (pad[0] = 0) are uint64 with checked
+// arithmetic.  Bound by memory traffic: a width-18 job's arena is 1.3 MB and 1536 of them are
+// in flight, far beyond the caches.  n=100, m=300 over 46816 cubes of width 18 (23 G elements
+// read and written): 84 ms with uint64 tensors and one thread per output, 66 ms with uint32
+// ones (the longest sums of 2^16 terms on one thread then hold their job for 40 ms), 51 ms
+// with long sums shared out over a wave and the jobs taken longest first.
+struct CountTag {
+  uint32_t v;
+  __device__ uint32_t lhs() const { return v & 3u; }          // 0 uint64, 1 uint32, 2 uint64 below 2^32
+  __device__ uint32_t rhs() const { return (v >> 2) & 3u; }
+  __device__ bool out32() const { return v & TS_COUNT_OUT32; }
+  __device__ bool exact() const { return v & TS_COUNT_EXACT; }  // no sum or product reaches 2^64
+};
+
+constexpr int CWG = 256;  // threads of a counting workgroup (512: 51 ms too, 1024: 72)
+constexpr int K64 = 0, K32 = 1, KLOW = 2, KNONE = 3;
+
+// The 2^NC contiguous entries of one row (element offset `at` of a tensor at `base`).
+template <int K, int NC>
+struct CountRow {
+  uint64_t v[1 << NC];
+};
+template <int K, int NC>
+__device__ __forceinline__ CountRow<K, NC> count_row(const uint8_t* base, uint32_t at) {
+  CountRow<K, NC> r;
+  if constexpr (K == KNONE) {
+#pragma unroll
+    for (int c = 0; c < (1 << NC); ++c) r.v[c] = 1;
+  } else if constexpr (K == K32) {
+    const uint8_t* p = base + 4u * at;
+    if constexpr (NC == 0) {
+      r.v[0] = *reinterpret_cast<const uint32_t*>(p);
+    } else if constexpr (NC == 1) {
+      const uint2 x = *reinterpret_cast<const uint2*>(p);
+      r.v[0] = x.x;
+      r.v[1] = x.y;
+    } else {
+      const uint4 x = *reinterpret_cast<const uint4*>(p);
+      r.v[0] = x.x;
+      r.v[1] = x.y;
+      r.v[2] = x.z;
+      r.v[3] = x.w;
+    }
+  } else {
+    const uint8_t* p = base + 8u * at;
+    uint2 x[1 << NC];
+    if constexpr (NC == 0) {
+      x[0] = *reinterpret_cast<const uint2*>(p);
+    } else {
+#pragma unroll
+      for (int h = 0; h < (1 << NC) / 2; ++h) {
+        const uint4 y = reinterpret_cast<const uint4*>(p)[h];
+        x[2 * h] = make_uint2(y.x, y.y);
+        x[2 * h + 1] = make_uint2(y.z, y.w);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < (1 << NC); ++c) r.v[c] = K == KLOW ? (uint64_t)x[c].x : ((uint64_t)x[c].y << 32) | x[c].x;
+  }
+  return r;
+}
+
+// One step of at most 4 contiguous terms per output: U outputs per thread and trip (outputs
+// tid, 256 + tid, ... of a run of 256 U), all their rows loaded before any is used.
+template <int KL, int KR, int NC>
+__device__ __forceinline__ void count_rows(const ts_step& st, const Lut& L, const uint8_t* lhs, const uint8_t* rhs,
+                                           uint8_t* out, bool out32, uint32_t lo_l, uint32_t lo_r, int nqo, int tid) {
+  constexpr int ROW = ((KL == K32 ? 4 : 8) + (KR == K32 ? 4 : KR == KNONE ? 0 : 8)) << NC;  // bytes per output
+  constexpr int U = ROW <= 16 ? 4 : 2;
+  const uint32_t n = 1u << st.out_rank;
+  for (uint32_t b0 = 0; b0 < n; b0 += CWG * U) {
+    CountRow<KL, NC> a[U];
+    CountRow<KR, NC> b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t o = b0 + u * CWG + tid;
+      if (o < n) {
+        const uint32_t hi = o >> 8;
+        a[u] = count_row<KL, NC>(lhs, lo_l + hi_off<4>(L.ol, hi, nqo));
+        b[u] = count_row<KR, NC>(rhs, lo_r + hi_off<4>(L.orr, hi, nqo));
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t o = b0 + u * CWG + tid;
+      if (o < n) {
+        uint64_t acc = 0;
+#pragma unroll
+        for (int c = 0; c < (1 << NC); ++c) {
+          if constexpr (KR == KNONE) acc += a[u].v[c];
+          else if constexpr (KL == K64 || KR == K64) acc += a[u].v[c] * b[u].v[c];
+          else acc += (uint64_t)(uint32_t)a[u].v[c] * (uint32_t)b[u].v[c];
+        }
+        if (out32) reinterpret_cast<uint32_t*>(out)[o] = (uint32_t)acc;
+        else reinterpret_cast<uint64_t*>(out)[o] = acc;
+      }
+    }
+  }
+}
+
+template <int KL, int KR>
+__device__ __forceinline__ void count_rows_nc(const ts_step& st, const Lut& L, const uint8_t* lhs, const uint8_t* rhs,
+                                              uint8_t* out, bool out32, uint32_t lo_l, uint32_t lo_r, int nqo, int tid) {
+  if (st.sum_rank == 0) count_rows<KL, KR, 0>(st, L, lhs, rhs, out, out32, lo_l, lo_r, nqo, tid);
+  else if (st.sum_rank == 1) count_rows<KL, KR, 1>(st, L, lhs, rhs, out, out32, lo_l, lo_r, nqo, tid);
+  else count_rows<KL, KR, 2>(st, L, lhs, rhs, out, out32, lo_l, lo_r, nqo, tid);
+}
+
+template <int KL>
+__device__ __forceinline__ void count_rows_r(uint32_t kr, const ts_step& st, const Lut& L, const uint8_t* lhs,
+                                             const uint8_t* rhs, uint8_t* out, bool out32, uint32_t lo_l, uint32_t lo_r,
+                                             int nqo, int tid) {
+  if (kr == K64) count_rows_nc<KL, K64>(st, L, lhs, rhs, out, out32, lo_l, lo_r, nqo, tid);
+  else if (kr == K32) count_rows_nc<KL, K32>(st, L, lhs, rhs, out, out32, lo_l, lo_r, nqo, tid);
+  else if (kr == KLOW) count_rows_nc<KL, KLOW>(st, L, lhs, rhs, out, out32, lo_l, lo_r, nqo, tid);
+  else count_rows_nc<KL, KNONE>(st, L, lhs, rhs, out, out32, lo_l, lo_r, nqo, tid);
+}
+
+__device__ __forceinline__ uint64_t shfl_xor64(uint64_t x, int m) {
+  return ((uint64_t)(uint32_t)__shfl_xor((int)(x >> 32), m) << 32) | (uint32_t)__shfl_xor((int)(uint32_t)x, m);
+}
+
+// Steps of 8 or more contiguous terms per output, tables built: 2^pb lanes per output (at
+// most a wave), each taking every 2^pb-th block of 4 terms, so neighbouring lanes read
+// neighbouring blocks and a scalar closing a tree is no serial walk over its terms.
+template <int KL, int KR>
+__device__ __forceinline__ void count_long(const ts_step& st, const Lut& L, const uint8_t* lhs, const uint8_t* rhs,
+                                           uint8_t* out, bool out32, int tid) {
+  constexpr int V = 2;  // blocks in flight per lane
+  const int nqo = nchunks(st.out_rank), pb = min(st.sum_rank - 2, 6);
+  const uint32_t n = 1u << st.out_rank, nblk = 1u << (st.sum_rank - 2), P = 1u << pb;
+  const uint32_t p = tid & (P - 1);
+  for (uint32_t o0 = 0; o0 < n; o0 += CWG >> pb) {
+    const uint32_t o = o0 + (tid >> pb);
+    uint64_t acc = 0;
+    if (o < n) {
+      const uint32_t offl = c_off<4>(L.ol, o, nqo), offr = c_off<4>(L.orr, o, nqo);
+      for (uint32_t k = p; k < nblk; k += V * P) {
+        CountRow<KL, 2> a[V];
+        CountRow<KR, 2> b[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+          if (k + v * P < nblk) {
+            a[v] = count_row<KL, 2>(lhs, offl + 4 * (k + v * P));
+            b[v] = count_row<KR, 2>(rhs, offr + 4 * (k + v * P));
+          }
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+          if (k + v * P < nblk)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc += a[v].v[c] * b[v].v[c];
+      }
+    }
+    for (int m = 1; m < (int)P; m <<= 1) acc += shfl_xor64(acc, m);
+    if (o < n && p == 0) {
+      if (out32) reinterpret_cast<uint32_t*>(out)[o] = (uint32_t)acc;
+      else reinterpret_cast<uint64_t*>(out)[o] = acc;
+    }
+  }
+}
+
+template <int KL>
+__device__ __forceinline__ void count_long_r(uint32_t kr, const ts_step& st, const Lut& L, const uint8_t* lhs,
+                                             const uint8_t* rhs, uint8_t* out, bool out32, int tid) {
+  if (kr == K64) count_long<KL, K64>(st, L, lhs, rhs, out, out32, tid);
+  else if (kr == K32) count_long<KL, K32>(st, L, lhs, rhs, out, out32, tid);
+  else if (kr == KLOW) count_long<KL, KLOW>(st, L, lhs, rhs, out, out32, tid);
+  else count_long<KL, KNONE>(st, L, lhs, rhs, out, out32, tid);
+}
+
+// Any other step, tables built: terms one by one, each output's shared out over 2^pb lanes of
+// a wave, sums and products checked.  Returns true if a value overflowed.
+__device__ inline bool count_general(const ts_step& st, CountTag tag, const Lut& L, const uint8_t* lhs,
+                                     const uint8_t* rhs, uint8_t* out, int tid) {
+  const int nc = st.sum_rank, nqo = nchunks(st.out_rank), nqc = nchunks(nc);
+  const bool norhs = st.flags & TS_STEP_NORHS, kinner = st.flags & TS_STEP_KINNER;
+  const bool l32 = tag.lhs() == K32, r32 = tag.rhs() == K32, out32 = tag.out32();
+  const int pb = min(nc, 6);
+  const uint32_t n = 1u << st.out_rank, nterm = 1u << nc, P = 1u << pb, p = tid & (P - 1);
+  bool ovf = false;
+  for (uint32_t o0 = 0; o0 < n; o0 += CWG >> pb) {
+    const uint32_t o = o0 + (tid >> pb);
+    uint64_t acc = 0;
+    if (o < n) {
+      const uint32_t offl = c_off<4>(L.ol, o, nqo), offr = c_off<4>(L.orr, o, nqo);
+      for (uint32_t c = p; c < nterm; c += P) {
+        const uint32_t il = offl + (kinner ? c : c_off<4>(L.cl, c, nqc));
+        const uint32_t ir = offr + (kinner ? c : c_off<4>(L.cr, c, nqc));
+        const uint64_t a = l32 ? reinterpret_cast<const uint32_t*>(lhs)[il] : reinterpret_cast<const uint64_t*>(lhs)[il];
+        uint64_t b = 1;
+        if (!norhs) b = r32 ? reinterpret_cast<const uint32_t*>(rhs)[ir] : reinterpret_cast<const uint64_t*>(rhs)[ir];
+        uint64_t x;
+        ovf |= __builtin_mul_overflow(a, b, &x);
+        ovf |= __builtin_add_overflow(acc, x, &acc);
+      }
+    }
+    for (int m = 1; m < (int)P; m <<= 1) ovf |= __builtin_add_overflow(acc, shfl_xor64(acc, m), &acc);
+    if (o < n && p == 0) {
+      if (out32) reinterpret_cast<uint32_t*>(out)[o] = (uint32_t)acc;
+      else reinterpret_cast<uint64_t*>(out)[o] = acc;
+    }
+  }
+  return ovf;
+}
+
+// arena_stride is in bytes; each job's scalar result times 2^free_vars is added to its
 // instance's count; any overflow sets the instance's flag.
-__global__ __launch_bounds__(WG) void k_batch_count(ts_batch b, unsigned long long* __restrict__ counts,
+__global__ __launch_bounds__(CWG) void k_batch_count(ts_batch b, unsigned long long* __restrict__ counts,
                                                     int32_t* __restrict__ overflow) {
   __shared__ Lut L;
   __shared__ ts_step s_steps[SREC];
@@ -496,21 +705,54 @@ __global__ __launch_bounds__(WG) void k_batch_count(ts_batch b, unsigned long lo
     const ts_job job = b.jobs[j];
     {
       const uint8_t* src = b.leaves + job.leaf_begin;
-      for (int i = tid; i < job.num_leaf_bytes; i += WG) arena[i] = src[i];
+      for (int i = tid; i < job.num_leaf_bytes; i += CWG) arena[i] = src[i];
     }
     bool ovf = false;
     for (int s0 = 0; s0 < job.num_steps; s0 += SREC) {
       const int ns = min(SREC, job.num_steps - s0);
       const uint4* src = reinterpret_cast<const uint4*>(b.steps + job.step_begin + s0);
-      for (int i = tid; i < ns * 8; i += WG) reinterpret_cast<uint4*>(s_steps)[i] = src[i];
+      for (int i = tid; i < ns * 8; i += CWG) reinterpret_cast<uint4*>(s_steps)[i] = src[i];
       __syncthreads();
       for (int s = 0; s < ns; ++s) {
         const ts_step& st = s_steps[s];
-        const bool need_c = !(st.flags & TS_STEP_KINNER) && st.sum_rank > 0;
-        build_lut(st, L, need_c, tid);
-        __syncthreads();
-        const uint64_t* rhs = arena + ((st.flags & TS_STEP_NORHS) ? st.lhs_off : st.rhs_off);
-        ovf |= step_u64(st, L, arena + st.lhs_off, rhs, arena + st.out_off, (uint64_t)tid, (uint64_t)WG);
+        const CountTag tag{st.pad[0]};
+        const bool kinner = st.flags & TS_STEP_KINNER, norhs = st.flags & TS_STEP_NORHS;
+        uint8_t* base = reinterpret_cast<uint8_t*>(arena);
+        const uint8_t* lhs = base + 8ull * st.lhs_off;
+        const uint8_t* rhs = base + 8ull * (norhs ? st.lhs_off : st.rhs_off);
+        uint8_t* out = base + 8ull * st.out_off;
+        const uint32_t kl = tag.lhs(), kr = norhs ? (uint32_t)KNONE : tag.rhs();
+        const bool rows = tag.exact() && (kinner || st.sum_rank == 0);
+        if (rows && st.sum_rank <= 2) {
+          uint32_t lo_l = 0, lo_r = 0;
+          int nqo = 1;
+          if (st.out_rank <= 8) {  // one output per thread, its offsets straight from the record
+            for (int j = 0; j < st.out_rank; ++j)
+              if ((tid >> j) & 1) {
+                if (st.o_lpos[j] != TS_NOPOS) lo_l |= 1u << st.o_lpos[j];
+                if (st.o_rpos[j] != TS_NOPOS) lo_r |= 1u << st.o_rpos[j];
+              }
+          } else {
+            build_lut(st, L, false, tid);
+            __syncthreads();
+            nqo = nchunks(st.out_rank);
+            lo_l = L.ol[0][tid & 255];
+            lo_r = L.orr[0][tid & 255];
+          }
+          if (kl == K64) count_rows_r<K64>(kr, st, L, lhs, rhs, out, tag.out32(), lo_l, lo_r, nqo, tid);
+          else if (kl == K32) count_rows_r<K32>(kr, st, L, lhs, rhs, out, tag.out32(), lo_l, lo_r, nqo, tid);
+          else count_rows_r<KLOW>(kr, st, L, lhs, rhs, out, tag.out32(), lo_l, lo_r, nqo, tid);
+        } else if (rows) {
+          build_lut(st, L, false, tid);
+          __syncthreads();
+          if (kl == K64) count_long_r<K64>(kr, st, L, lhs, rhs, out, tag.out32(), tid);
+          else if (kl == K32) count_long_r<K32>(kr, st, L, lhs, rhs, out, tag.out32(), tid);
+          else count_long_r<KLOW>(kr, st, L, lhs, rhs, out, tag.out32(), tid);
+        } else {
+          build_lut(st, L, !kinner && st.sum_rank > 0, tid);
+          __syncthreads();
+          ovf |= count_general(st, tag, L, lhs, rhs, out, tid);
+        }
         __syncthreads();
       }
     }
@@ -630,7 +872,7 @@ int ts_batch_count(const ts_batch* b, uint64_t* counts, int32_t* overflow, ts_st
   if (b->num_jobs > 0 && (!b->jobs || !b->steps || !b->leaves || !b->arenas)) return TS_EINVAL;
   if (b->arena_stride <= 0 || (b->arena_stride & 255)) return TS_EINVAL;
   if (b->num_jobs == 0) return TS_OK;
-  hipLaunchKernelGGL(k_batch_count, dim3(b->num_workgroups), dim3(WG), 0, reinterpret_cast<hipStream_t>(stream),
+  hipLaunchKernelGGL(k_batch_count, dim3(b->num_workgroups), dim3(CWG), 0, reinterpret_cast<hipStream_t>(stream),
                      *b, reinterpret_cast<unsigned long long*>(counts), overflow);
   return hipGetLastError() == hipSuccess ? TS_OK : TS_EHIP;
 }

@@ -187,6 +187,100 @@ extern "C" int tsc_packetize(ts_job* jobs, int64_t num_jobs, ts_step* steps, int
   return TSP_OK;
 }
 
+// ---- counting widths --------------------------------------------------------------
+
+namespace {
+
+struct Held {  // the tensor at an arena offset
+  uint32_t off;
+  int rank, bound, kind, step;  // step: the one that wrote it (-1: a leaf)
+};
+
+// One job's tags; false if an operand is not a whole tensor written before.
+bool count_widths_job(const ts_job& job, ts_step* st, const uint8_t* leaves, std::vector<Held>& table,
+                      std::vector<uint8_t>& tags) {
+  const int n = job.num_steps;
+  size_t cap = 64;
+  while (cap < 4u * (size_t)(n + 1)) cap *= 2;
+  table.assign(cap, Held{UINT32_MAX, 0, 0, 0, 0});
+  auto slot = [&](uint32_t off) -> Held& {
+    size_t h = (off * 0x9e3779b1u) & (cap - 1);
+    while (table[h].off != UINT32_MAX && table[h].off != off) h = (h + 1) & (cap - 1);
+    return table[h];
+  };
+  int leaf_bits = 0;
+  for (int32_t i = 0; i < job.num_leaf_bytes; ++i)
+    if (leaves[job.leaf_begin + i] > 1) leaf_bits = 8;
+  tags.assign(n, 0);
+  for (int i = 0; i < n; ++i) {
+    const ts_step& s = st[i];
+    int bound = s.sum_rank, kinds[2] = {0, 0};
+    for (int side = 0; side < ((s.flags & TS_STEP_NORHS) ? 1 : 2); ++side) {
+      const uint32_t off = side ? s.rhs_off : s.lhs_off;
+      const int rank = side ? s.rhs_rank : s.lhs_rank;
+      const Held& h = slot(off);
+      if (h.off == off) {
+        if (h.rank != rank) return false;
+        bound += h.bound;
+        kinds[side] = h.kind;
+      } else {
+        if ((uint64_t)off + (1ull << rank) > (uint64_t)job.num_leaf_bytes) return false;
+        bound += leaf_bits;
+        kinds[side] = 2;  // leaves are copied as uint64
+      }
+    }
+    // values up to 2^bound: uint32 holds 2^31, uint64 holds 2^63
+    const bool narrow = bound <= 31, exact = bound <= 63;
+    tags[i] = (uint8_t)(kinds[0] | (kinds[1] << 2) | (narrow ? TS_COUNT_OUT32 : 0) | (exact ? TS_COUNT_EXACT : 0));
+    slot(s.out_off) = Held{s.out_off, s.out_rank, bound, narrow ? 1 : 0, i};
+  }
+  // The result is read as uint64; it is the last tensor at its offset, so no step reads it.
+  const Held& res = slot((uint32_t)job.result_off);
+  if (res.off == (uint32_t)job.result_off) {
+    if (res.rank != job.result_rank) return false;
+    for (int i = res.step + 1; i < n; ++i)
+      if (st[i].lhs_off == res.off || (!(st[i].flags & TS_STEP_NORHS) && st[i].rhs_off == res.off)) return false;
+    tags[res.step] &= (uint8_t)~TS_COUNT_OUT32;
+  }
+  return true;
+}
+
+}  // namespace
+
+extern "C" int tsc_count_widths(const ts_job* jobs, int64_t num_jobs, ts_step* steps, int64_t num_steps,
+                                const uint8_t* leaves, int64_t num_leaf_bytes, int32_t threads) {
+  if (num_jobs < 0 || num_steps < 0 || num_leaf_bytes < 0 || (num_jobs > 0 && !jobs) || (num_steps > 0 && !steps) ||
+      (num_leaf_bytes > 0 && !leaves))
+    return TSP_EINVAL;
+  for (int64_t j = 0; j < num_jobs; ++j)
+    if (jobs[j].step_begin < 0 || jobs[j].num_steps < 0 || (int64_t)jobs[j].step_begin + jobs[j].num_steps > num_steps ||
+        jobs[j].leaf_begin < 0 || jobs[j].num_leaf_bytes < 0 ||
+        jobs[j].leaf_begin + jobs[j].num_leaf_bytes > num_leaf_bytes)
+      return TSP_EINVAL;
+  // Jobs that share step records must agree on their tags: such programs stay uint64.
+  for (int64_t i = 0; i < num_steps; ++i) steps[i].pad[0] = 0;
+  std::vector<uint8_t> used((size_t)num_steps, 0);
+  for (int64_t j = 0; j < num_jobs; ++j)
+    for (int32_t i = 0; i < jobs[j].num_steps; ++i)
+      if (used[jobs[j].step_begin + i]++) return TSP_OK;
+  int nt = threads > 0 ? threads : (int)std::max(1u, std::thread::hardware_concurrency());
+  nt = (int)std::max<int64_t>(1, std::min<int64_t>(nt, num_jobs / 64 + 1));
+  auto work = [&](int t) {
+    std::vector<Held> table;
+    std::vector<uint8_t> tags;
+    for (int64_t j = t; j < num_jobs; j += nt) {
+      ts_step* st = steps + jobs[j].step_begin;
+      if (!count_widths_job(jobs[j], st, leaves, table, tags)) continue;
+      for (int32_t i = 0; i < jobs[j].num_steps; ++i) st[i].pad[0] = tags[i];
+    }
+  };
+  std::vector<std::thread> pool;
+  for (int t = 1; t < nt; ++t) pool.emplace_back(work, t);
+  work(0);
+  for (auto& th : pool) th.join();
+  return TSP_OK;
+}
+
 // ---- lane form ------------------------------------------------------------------
 
 static_assert(sizeof(ts_lane) == 16, "one uint4 per lane record");

@@ -436,7 +436,7 @@ class BatchCounter:
     def __init__(self, prog: Program, *, num_workgroups: int | None = None, device: str = "cuda") -> None:
         torch = _torch()
         L = N.lib()
-        self.dp = DeviceProgram(prog, device)
+        self.dp = DeviceProgram(PG.count_widths(prog), device)
         self.prog = prog
         nj = len(prog.jobs)
         if num_workgroups is None:
@@ -449,7 +449,9 @@ class BatchCounter:
         num_workgroups = min(int(num_workgroups), max(N.BATCH_SEGMENTS, ARENA_BUDGET // self.arena_stride))
         self.num_workgroups = max(1, min(max(num_workgroups, N.BATCH_SEGMENTS), max(1, nj)))
         self.arenas = torch.empty(self.num_workgroups * self.arena_stride, dtype=torch.uint8, device=device)
-        self.order = torch.from_numpy(dispatch_order(prog)).to(device)
+        # Every job runs (no early exit): longest first, so the queue drains on short ones.
+        order = np.argsort(-job_work(prog), kind="stable").astype(np.int32)
+        self.order = torch.from_numpy(order).to(device)
         n = max(1, prog.num_instances)
         self.counts = torch.zeros(n, dtype=torch.int64, device=device)
         self.overflow = torch.zeros(n, dtype=torch.int32, device=device)

@@ -93,6 +93,8 @@ def _lib():
                                       ctypes.c_int32, vp, ctypes.c_int64, P(ctypes.c_int64)]
         L.tsc_search_plan.restype = ctypes.c_int
         L.tsc_lanes.argtypes = [vp, ctypes.c_int64, vp, ctypes.c_int64, vp, ctypes.c_int64, vp, ctypes.c_int32]
+        L.tsc_count_widths.argtypes = [vp, ctypes.c_int64, vp, ctypes.c_int64, vp, ctypes.c_int64, ctypes.c_int32]
+        L.tsc_count_widths.restype = ctypes.c_int
         for f in (L.tsc_compile, L.tsc_sat_batch, L.tsc_program_sizes, L.tsc_program_copy, L.tsp_elim,
                   L.tsp_elim_order, L.tsp_order_cost, L.tsp_elim_order_prior, L.tsc_packetize, L.tsc_lanes):
             f.restype = ctypes.c_int
@@ -406,6 +408,19 @@ def packetize(prog: Program, threads: int = 0) -> Program:
     out = Program(jobs, steps, prog.leaves, prog.stats, dict(prog.meta))
     out.meta["packetized"] = True
     return out
+
+
+def count_widths(prog: Program, threads: int = 0) -> Program:
+    """
+    ``prog`` with the storage width of every counting step in its record
+    (``tsc_count_widths``): tensors whose entries are provably below 2^32 are held as
+    uint32 by the batched counter.  Values are unchanged; returns a new Program.
+    """
+    steps = prog.steps.copy()
+    leaves = np.ascontiguousarray(prog.leaves, dtype=np.uint8)
+    _plan._check(_lib().tsc_count_widths(prog.jobs.ctypes.data, len(prog.jobs), steps.ctypes.data, len(steps),
+                                         leaves.ctypes.data, leaves.size, int(threads)), "tsc_count_widths")
+    return Program(prog.jobs, steps, prog.leaves, prog.stats, dict(prog.meta))
 
 
 LANE_DTYPE = np.dtype(

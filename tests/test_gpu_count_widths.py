@@ -1,0 +1,105 @@
+"""
+Counting with narrow storage: the widths written into the step records (CPU), and exact counts
+on the GPU at the edges of uint32 and uint64 (products of disjoint clauses have closed forms).
+"""
+
+import numpy as np
+import pytest
+
+from oracle import brute
+from tensorsat_amd import program as PG
+from tensorsat_amd.network import Wiring
+from tensorsat_amd.sat import CNFInstance
+
+OUT32, EXACT = 16, 32
+
+
+def _bounds(prog, job):
+    """(bound bits, lhs kind, rhs kind) per step of a job, by following arena offsets."""
+    held = {}
+    for st in prog.steps[job["step_begin"] : job["step_begin"] + job["num_steps"]]:
+        sides = [int(st["lhs_off"])] + ([] if st["flags"] & PG.STEP_NORHS else [int(st["rhs_off"])])
+        parts = [held.get(o, (0, 2)) for o in sides]
+        b = sum(p[0] for p in parts) + int(st["sum_rank"])
+        yield b, parts[0][1], parts[1][1] if len(parts) > 1 else 0
+        held[int(st["out_off"])] = (b, 1 if b <= 31 else 0)
+
+
+def _check_tags(prog):
+    got = PG.count_widths(prog)
+    seen = set()
+    for job in got.jobs:
+        steps = got.steps[job["step_begin"] : job["step_begin"] + job["num_steps"]]
+        last = [int(o) for o in steps["out_off"]]
+        final = len(last) - 1 - last[::-1].index(int(job["result_off"])) if int(job["result_off"]) in last else -1
+        for i, (st, (b, kl, kr)) in enumerate(zip(steps, _bounds(prog, job))):
+            want = kl | kr << 2 | (EXACT if b <= 63 else 0) | (OUT32 if b <= 31 and i != final else 0)
+            assert int(st["pad"][0]) == want, (i, b)
+            seen.add(want & (OUT32 | EXACT))
+    assert not prog.steps["pad"].any()  # the given program is left alone
+    return seen
+
+
+def _disjoint(m):
+    """m clauses on 3 variables each, as one job: 7^m models, 3 m summed bits."""
+    w = Wiring([2] * (3 * m), [[3 * i, 3 * i + 1, 3 * i + 2] for i in range(m)], [])
+    leaf = np.ones((2, 2, 2), np.uint8)
+    leaf[1, 0, 1] = 0
+    return PG.compile_network(w, [leaf] * m, PG.elim(w, trials=1))
+
+
+def test_widths_follow_the_summed_bits():
+    cnfs = [CNFInstance.random(3, n, 3 * n, rng=n) for n in (12, 30, 44)]
+    assert _check_tags(PG.sat_batch(cnfs, width=10)) == {OUT32 | EXACT, EXACT}
+    for m, kinds in ((10, {OUT32 | EXACT, EXACT}), (21, {OUT32 | EXACT, EXACT}), (23, {OUT32 | EXACT, EXACT, 0})):
+        assert _check_tags(_disjoint(m)) == kinds
+
+
+def test_leaf_bytes_above_one_and_shared_records():
+    w = Wiring([2] * 3, [[0, 1], [1, 2]], [])
+    prog = PG.compile_network(w, [np.ones((2, 2), np.uint8)] * 2, PG.elim(w, trials=1))
+    narrow = PG.count_widths(prog).steps["pad"][:, 0]
+    prog.leaves[0] = 200  # 8 bits per leaf: 16 + 3 summed
+    assert (PG.count_widths(prog).steps["pad"][:, 0] == narrow).all()
+    two = PG.concat([prog], [np.zeros(1, np.int64)], 1)
+    two.jobs = np.concatenate([two.jobs, two.jobs])  # both jobs run the same records
+    assert not PG.count_widths(two).steps["pad"].any()
+
+
+@pytest.mark.gpu
+def test_counts_at_the_edges_of_the_widths():
+    from tensorsat_amd.executor import BatchCounter
+
+    for m in (1, 9, 10, 11, 20, 21, 22):  # 7^22 < 2^62, a bound of 66 bits: checked arithmetic
+        assert BatchCounter(_disjoint(m)).run() == [7**m], m
+    with pytest.raises(OverflowError):
+        BatchCounter(_disjoint(23)).run()  # 7^23 > 2^64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,width", [(14, 3), (20, 9), (22, 12), (24, 16)])
+def test_counts_match_brute_force(n, width):
+    from tensorsat_amd.executor import BatchCounter
+
+    cnfs = [CNFInstance.random(3, n, int(r * n), rng=40 * n + i) for i, r in enumerate((1.0, 2.0, 3.0))]
+    got = BatchCounter(PG.sat_batch(cnfs, width=width)).run()
+    assert got == [brute.count(c.num_vars, c.clauses) for c in cnfs]
+
+
+@pytest.mark.gpu
+def test_wide_sums_and_general_steps():
+    """A step of 2 out bits that is not K-innermost, and one summing 8 bits at once."""
+    from tensorsat_amd.executor import BatchCounter
+    from wide_steps import wide_sum_program
+
+    for permute in (True, False):
+        prog, leaves = wide_sum_program(3, out_wires=(), n=10, density=0.5, permute=permute)
+        got = BatchCounter(prog).run()
+        off = [int(prog.steps["lhs_off"][0]), int(prog.steps["rhs_off"][0])]
+        lhs, rhs = (prog.leaves[o : o + 1024].astype(np.int64) for o in off)
+        idx = np.arange(1024)
+        at = [np.zeros(1024, np.int64), np.zeros(1024, np.int64)]
+        for k in range(10):
+            for side, name in enumerate(("c_lpos", "c_rpos")):
+                at[side] |= ((idx >> k) & 1) << int(prog.steps[name][0, k])
+        assert got == [int((lhs[at[0]] * rhs[at[1]]).sum())]
