@@ -399,6 +399,14 @@ int ts_gnn_gemm(const void* A, int64_t sam, int64_t sak, const void* B, int64_t 
                 int64_t ldc, int32_t M, int32_t N, int32_t K, const float* bias, int32_t relu,
                 int32_t out_bf16, int32_t accumulate, ts_stream stream);
 
+/* dW[m*ldw + n] += sum over rows r of X[r*ldx + m] dZ[r*ldz + n] (bf16 in, fp32 out and sums):
+ * weight gradients.  N = 128 columns with 8-byte aligned rows go in one pass over X, partial
+ * sums through `scratch` (device memory, 16-byte aligned; ts_gnn_wgrad_scratch says how much
+ * the call can use); anything else, or less scratch, runs as ts_gnn_gemm. */
+int ts_gnn_wgrad_scratch(int32_t M, int32_t rows, int64_t* bytes);
+int ts_gnn_wgrad(const void* X, int64_t ldx, const void* dZ, int64_t ldz, int32_t M, int32_t N, int32_t rows,
+                 float* dW, int64_t ldw, void* scratch, int64_t scratch_bytes, ts_stream stream);
+
 /* Weighted signed neighbour sums over a CSR incidence (row r -> col[e], weight w[e] whose
  * sign is the literal's): forward writes sum |w| X[col, xoff..] over positive and negative
  * edges into bf16 column blocks off_pos / off_neg; with out_f32_accumulate both signs (read

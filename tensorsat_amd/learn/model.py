@@ -114,6 +114,23 @@ class GNN:
             out_b = M * Nn * (2 if out_bf16 else 4) * (2 if acc else 1)  # read back when accumulating
             log.append((2.0 * M * Nn * K, 2.0 * (M * K + K * Nn) + out_b, e0, e1))
 
+    def _wgrad(self, X, ldx, dZ, ldz, M, rows, dW):
+        """dW (fp32 [M, HID]) += X^T dZ over the rows; partial sums in scratch memory that
+        goes back to the allocator on this stream."""
+        torch = self.torch
+        need = N.i64(0)
+        N.check(N.lib().ts_gnn_wgrad_scratch(M, rows, N.ctypes.byref(need)), "ts_gnn_wgrad_scratch")
+        scratch = torch.empty(max(16, need.value), dtype=torch.uint8, device=self.device)
+        log = self.gemm_log
+        if log is not None:
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+        N.check(N.lib().ts_gnn_wgrad(X, ldx, dZ, ldz, M, HID, rows, dW, HID, N.dptr(scratch), need.value,
+                                     N.stream_ptr()), "ts_gnn_wgrad")
+        if log is not None:
+            e1.record()
+            log.append((2.0 * M * HID * rows, 2.0 * (M + HID) * rows + 8.0 * M * HID, e0, e1))
+
     def _segsum(self, rowptr, col, weight, nrows, X, ldx, xp, xn, xf32, out, ldo, op, on, acc):
         N.check(N.lib().ts_gnn_segsum(rowptr, col, weight, nrows, X, ldx, xp, xn, xf32, out, ldo, op, on, HID, acc,
                                       N.stream_ptr()), "ts_gnn_segsum")
@@ -175,8 +192,7 @@ class GNN:
             # variable update of layer l
             N.check(L.ts_gnn_relu_back(dHv.data_ptr(), HID, Xv[l + 1].data_ptr(), ld3, V, HID, dZv.data_ptr(), HID,
                                        self.gp(f"bv{l}"), s), "relu_back")
-            self._gemm(Xv[l].data_ptr(), 1, ld3, dZv.data_ptr(), HID, 1, self.gp(f"Wv{l}"), HID, ld3, HID, V,
-                       out_bf16=0, acc=1)
+            self._wgrad(Xv[l].data_ptr(), ld3, dZv.data_ptr(), HID, ld3, V, self.gp(f"Wv{l}"))
             dHv_new = torch.empty((max(V, 1), HID), dtype=torch.float32, device=dev)
             self._gemm(dZv.data_ptr(), HID, 1, self.bf(f"Wv{l}"), 1, HID, dHv_new.data_ptr(), HID, V, HID, HID,
                        out_bf16=0)
@@ -187,8 +203,7 @@ class GNN:
             # clause update of layer l
             N.check(L.ts_gnn_relu_back(dHc.data_ptr(), HID, Xc[l + 1].data_ptr(), ld3, C, HID, dZc.data_ptr(), HID,
                                        self.gp(f"bc{l}"), s), "relu_back")
-            self._gemm(Xc[l].data_ptr(), 1, ld3, dZc.data_ptr(), HID, 1, self.gp(f"Wc{l}"), HID, ld3, HID, C,
-                       out_bf16=0, acc=1)
+            self._wgrad(Xc[l].data_ptr(), ld3, dZc.data_ptr(), HID, ld3, C, self.gp(f"Wc{l}"))
             dHc_new = torch.empty((max(C, 1), HID), dtype=torch.float32, device=dev)
             self._gemm(dZc.data_ptr(), HID, 1, self.bf(f"Wc{l}"), 1, HID, dHc_new.data_ptr(), HID, C, HID, HID,
                        out_bf16=0)
@@ -200,12 +215,10 @@ class GNN:
         # input embeddings
         N.check(L.ts_gnn_relu_back(dHv.data_ptr(), HID, Xv[0].data_ptr(), ld3, V, HID, dZv.data_ptr(), HID,
                                    self.gp("b_vin"), s), "relu_back")
-        self._gemm(dg.var_feat.data_ptr(), 1, FEAT, dZv.data_ptr(), HID, 1, self.gp("W_vin"), HID, FEAT, HID, V,
-                   out_bf16=0, acc=1)
+        self._wgrad(dg.var_feat.data_ptr(), FEAT, dZv.data_ptr(), HID, FEAT, V, self.gp("W_vin"))
         N.check(L.ts_gnn_relu_back(dHc.data_ptr(), HID, Xc[0].data_ptr(), ld3, C, HID, dZc.data_ptr(), HID,
                                    self.gp("b_cin"), s), "relu_back")
-        self._gemm(dg.clause_feat.data_ptr(), 1, FEAT, dZc.data_ptr(), HID, 1, self.gp("W_cin"), HID, FEAT, HID, C,
-                   out_bf16=0, acc=1)
+        self._wgrad(dg.clause_feat.data_ptr(), FEAT, dZc.data_ptr(), HID, FEAT, C, self.gp("W_cin"))
 
     def adam_step(self, lr: float = 1e-3, b1: float = 0.9, b2: float = 0.999, eps: float = 1e-8, wd: float = 0.0):
         self.steps += 1
