@@ -153,6 +153,15 @@ int ts_program_run_fused(const ts_job* job_host, const ts_step* steps_host, cons
                          const uint8_t* leaves_dev, uint8_t* arena, int32_t mode, int32_t small_bits,
                          ts_stream stream);
 
+/* One job whose arena fits TS_SMALL_ARENA bytes in one launch of one workgroup: the leaves are
+ * given on the host as bits (leaf entry i is bit i % 32 of word i / 32, num_leaf_bytes of
+ * them, at most 28672), the 2^result_rank result bytes go to `result` (device).  The steps
+ * are the same records as ts_program_run's, on the host and on the device; TS_EUNSUPPORTED
+ * for larger jobs. */
+#define TS_SMALL_ARENA 65536
+int ts_program_run_small(const ts_job* job, const ts_step* steps, const ts_step* steps_dev,
+                         const uint32_t* leaf_bits, uint8_t* result, int32_t mode, ts_stream stream);
+
 /* As ts_program_run_fused for `count` jobs at once (jobs_host: their records, contiguous
  * on the host), job g in arena + g * arena_stride (arena_stride a multiple of 256 and at
  * least every job's arena_elems): the jobs advance phase by phase -- phase p is each

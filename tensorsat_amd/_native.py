@@ -22,6 +22,8 @@ TS_EUNSUPPORTED = -3
 TS_EOVERFLOW = -4
 TS_EHIP = -5
 BATCH_LDS_MAX = 65536
+SMALL_ARENA = 65536  # TS_SMALL_ARENA
+SMALL_LEAVES = 28672  # leaf entries of a job run in one launch
 SCRATCH_MIN_BITS = 12  # contractions without a tensor of this rank never take scratch memory
 BATCH_SEGMENTS = 8  # queue counters per dispatch (TS_BATCH_SEGMENTS)
 BATCH_COUNTER_STRIDE = 64  # int32s between queue counters (TS_BATCH_COUNTER_STRIDE)
@@ -40,6 +42,7 @@ EXPORTS = (
     "ts_gnn_segsum", "ts_gnn_relu_back",
     "ts_gnn_head", "ts_gnn_adam", "ts_gnn_cast_bf16", "ts_dense_config", "ts_dense_tiles", "ts_dense_tile_of",
     "ts_search_run", "ts_search_run_queue", "ts_search_decide_noalloc", "ts_program_run_fused", "ts_program_run_gang",
+    "ts_program_run_small",
 )
 
 _lib = None
@@ -86,6 +89,7 @@ def load() -> ctypes.CDLL:
         L.ts_program_run.argtypes = [vp, vp, vp, vp, i32, vp, vp, vp]
         L.ts_program_count.argtypes = [vp, vp, vp, vp, vp, vp, vp]
         L.ts_program_run_fused.argtypes = [vp, vp, vp, vp, vp, i32, i32, vp]
+        L.ts_program_run_small.argtypes = [vp, vp, vp, vp, vp, i32, vp]
         L.ts_program_run_gang.argtypes = [vp, i32, vp, vp, vp, vp, i64, vp, i32, i32, vp]
         L.ts_batch_run.argtypes = [P(Batch), vp]
         L.ts_batch_compact.argtypes = [vp, i32, vp, vp, vp, vp, vp]

@@ -10,6 +10,8 @@ trees by the cotengra cost model), optionally slicing wires down to a size targe
 cotengra's ``ContractionTree.contract`` does through ``_autoray.einsum`` (a wire is
 summed at the first node after which no other tensor and no out port holds it), OR-s
 (``+``) the slices, adds dangling out wires and rewires to the out wires.
+Small trees over host leaves run as one device job instead (:class:`SmallTree`: the same steps
+in one launch).
 :meth:`contract_program` compiles the whole tree for the device executor instead.
 """
 
@@ -19,9 +21,11 @@ import itertools
 
 import numpy as np
 
+from .. import _native
 from .. import plan as _plan
 from .. import program as _prog
 from ..network import Diagram, Wiring
+from ..rel import DeviceRel
 from .abc import Contraction
 
 
@@ -87,6 +91,77 @@ def tree_steps(wiring: Wiring, path: np.ndarray, drop=()):
     return steps, root_legs
 
 
+class SmallTree:
+    """
+    A whole tree as one device job (``ts_program_run_small``): its step records, laid out
+    once per contraction, and where each leaf entry of a diagram goes in the job's leaves.
+    The steps are the tree's (:func:`tree_steps`), so every intermediate has the values that
+    the walk gives it, in the compiler's layouts; the result is in out-wire order.
+    """
+
+    # Products per step above which a workgroup's 256 lanes are no longer ahead of a launch
+    # per step: a step of 2^14 products takes them about 4 us, the walk 35 us of host.
+    MAX_TERMS = 1 << 14
+
+    @classmethod
+    def build(cls, wiring: Wiring, tree: _plan.Plan) -> "SmallTree | None":
+        """None where the walk has to run: sliced trees, extents other than 2, repeated or
+        dangling wires, a single slot, or tensors that do not fit one workgroup."""
+        slots, outs = wiring.slot_wires_list, wiring.out_wires
+        if len(slots) < 2 or len(tree.sliced) or any(d != 2 for d in wiring.wire_dims):
+            return None
+        held = {w for ws in slots for w in ws}
+        if len(set(outs)) != len(outs) or not held.issuperset(outs) or any(len(set(ws)) != len(ws) for ws in slots):
+            return None
+        if sum(1 << len(ws) for ws in slots) > _native.SMALL_LEAVES:
+            return None
+        cost = _plan.tree_cost(wiring, tree)
+        if cost.log2_max_size > 15:
+            return None
+        # The compiler lays leaf entries out in its own order: compiled with each entry's
+        # index (its low, then its high byte) as the value, the leaves say which goes where.
+        sizes = [1 << len(ws) for ws in slots]
+        index = np.split(np.arange(sum(sizes)), np.cumsum(sizes)[:-1])
+        lo, hi = (_prog.compile_network(wiring, [((ix >> sh) & 255).astype(np.uint8) for ix in index], tree)
+                  for sh in (0, 8))
+        terms = np.ldexp(1.0, lo.steps["out_rank"].astype(int) + lo.steps["sum_rank"]).sum()
+        if (len(lo.jobs) != 1 or int(lo.jobs["arena_elems"][0]) > _native.SMALL_ARENA or
+                lo.leaves.size > _native.SMALL_LEAVES or terms > cls.MAX_TERMS * len(lo.steps)):
+            return None
+        self = object.__new__(cls)
+        self.prog = lo
+        self.source = lo.leaves.astype(np.int64) | (hi.leaves.astype(np.int64) << 8)
+        self.shapes = [(2,) * len(ws) for ws in slots]
+        self.rank = len(outs)
+        self.device_steps = {}
+        return self
+
+    def leaf_bits(self, blocks) -> np.ndarray | None:
+        """The job's leaves as bits, or None if the blocks are not 0/1 host arrays of the
+        slots' shapes."""
+        if not all(type(b) is np.ndarray for b in blocks) or [b.shape for b in blocks] != self.shapes:
+            return None
+        flat = np.concatenate([b.reshape(-1) for b in blocks])
+        if flat.dtype != np.uint8 or flat.max() > 1:
+            return None
+        return np.packbits(flat[self.source], bitorder="little")
+
+    def run(self, bits: np.ndarray, box_class, mode: str):
+        import torch
+
+        N = _native
+        L = N.lib()
+        dev = torch.cuda.current_device()
+        steps = self.device_steps.get(dev)
+        if steps is None:  # a synchronous upload: complete for every stream
+            steps = self.device_steps[dev] = torch.from_numpy(self.prog.steps.view(np.uint8)).cuda()
+        res = torch.empty(max(16, 1 << self.rank), dtype=torch.uint8, device="cuda")
+        N.check(L.ts_program_run_small(N.host_ptr(self.prog.jobs), N.host_ptr(self.prog.steps), N.dptr(steps),
+                                       N.host_ptr(bits), N.dptr(res), N.MODES[mode], N.stream_ptr()),
+                "ts_program_run_small")
+        return box_class._new(res, (2,) * self.rank)
+
+
 class PlannedContraction(Contraction):
     """A contraction along a planned binary tree (``CotengraContraction`` counterpart)."""
 
@@ -100,6 +175,7 @@ class PlannedContraction(Contraction):
         if slicing_target is not None and tree.cost is not None and tree.cost.log2_max_size > slicing_target:
             tree = _plan.slice_plan(wiring, tree, slicing_target, reconfigure_trials=trials, seed=seed)
         self._tree = tree
+        self._small = False  # SmallTree or None, built on the first contraction
 
     @property
     def tree(self) -> _plan.Plan:
@@ -154,6 +230,12 @@ class PlannedContraction(Contraction):
     def contract(self, diagram: Diagram, *, order=None, autojit="auto", progbar: bool = False):
         """Validate and contract (``cotengra.py:100-128``)."""
         self.validate(diagram)
+        if self.box_class is DeviceRel:
+            if self._small is False:
+                self._small = SmallTree.build(self.wiring, self._tree)
+            bits = self._small.leaf_bits(diagram.blocks) if self._small is not None else None
+            if bits is not None:
+                return self._small.run(bits, DeviceRel, DeviceRel._mode)
         boxes = self._boxes(diagram)
         sliced = list(self._tree.sliced)
         dims = self.wiring.wire_dims

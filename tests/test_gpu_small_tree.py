@@ -1,0 +1,107 @@
+"""
+Trees that run as one device job (host leaves, every tensor in one workgroup's LDS) against
+the walk node by node and the oracle, and the diagrams that have to take the walk.
+"""
+
+import numpy as np
+import pytest
+
+from oracle_box import OracleRel
+from tensorsat_amd.contractions import PlannedContraction
+from tensorsat_amd.contractions.planned import SmallTree
+from tensorsat_amd.network import Diagram, Wiring
+from tensorsat_amd.sat import CNFInstance
+
+
+def _cnf_diagram(n, ratio, seed, inputs=None):
+    cnf = CNFInstance.random(3, n, int(round(ratio * n)), rng=seed)
+    return (cnf.inputs("_" * n if inputs is None else inputs) >> cnf.diagram()).flatten()
+
+
+def _random_diagram(rng, slots, wires, outs, rank=4):
+    ws = [[int(w) for w in rng.choice(wires, size=int(rng.integers(1, rank + 1)), replace=False)] for _ in range(slots)]
+    held = sorted({w for s in ws for w in s})
+    out = [int(w) for w in rng.permutation(held)[:outs]]
+    blocks = [(rng.random((2,) * len(s)) < 0.8).astype(np.uint8) for s in ws]
+    return Diagram(Wiring([2] * wires, ws, out), blocks)
+
+
+def test_trees_that_take_the_walk():
+    rng = np.random.default_rng(0)
+    leaf = np.ones((2, 2), np.uint8)
+
+    def small(*args, **kw):
+        w = Wiring(*args)
+        c = PlannedContraction(OracleRel, w, **kw)
+        return SmallTree.build(w, c.tree)
+
+    assert small([2] * 3, [[0, 1], [1, 2]], [0, 2]) is not None
+    assert small([3] * 3, [[0, 1], [1, 2]], [0, 2]) is None  # extents
+    assert small([2] * 3, [[0, 1, 2]], [0]) is None  # one slot
+    assert small([2] * 3, [[0, 0], [0, 1]], [1]) is None  # repeated wire in a slot
+    assert small([2] * 3, [[0, 1], [1, 2]], [0, 0]) is None  # repeated out wire
+    assert small([2] * 4, [[0, 1], [1, 2]], [3, 0]) is None  # dangling out wire
+    assert small([2] * 20, [[*range(0, 12)], [*range(8, 20)]], [*range(20)]) is None  # too large a result
+    t = small([2] * 3, [[0, 1], [1, 2]], [0, 2])
+    assert t.leaf_bits([leaf, leaf]) is not None
+    assert t.leaf_bits([leaf, leaf[0]]) is None and t.leaf_bits([leaf, 2 * leaf]) is None
+    assert t.leaf_bits([leaf, leaf.tolist()]) is None and t.leaf_bits([leaf, leaf.astype(np.int64)]) is None
+    # every leaf entry lands where the compiler puts it
+    d = _random_diagram(rng, 9, 8, 3)
+    s = SmallTree.build(d.wiring, PlannedContraction(OracleRel, d.wiring).tree)
+    from tensorsat_amd import program as PG
+
+    prog = PG.compile_network(d.wiring, list(d.blocks), PlannedContraction(OracleRel, d.wiring).tree)
+    assert (s.prog.steps == prog.steps).all()
+    got = np.unpackbits(s.leaf_bits(d.blocks), bitorder="little")[: prog.leaves.size]
+    for st in prog.steps:
+        for off, rank in ((st["lhs_off"], st["lhs_rank"]), (st["rhs_off"], st["rhs_rank"])):
+            if off < prog.jobs["num_leaf_bytes"][0] and off not in prog.steps["out_off"]:
+                assert (got[off : off + (1 << rank)] == prog.leaves[off : off + (1 << rank)]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["GT0", "MOD256"])
+def test_small_trees_match_the_walk_and_the_oracle(mode):
+    from tensorsat_amd.rel import DeviceRel
+
+    rng = np.random.default_rng(7)
+    diagrams = [_cnf_diagram(n, r, n) for n, r in ((3, 1.0), (6, 2.0), (9, 3.0), (10, 3.5), (12, 3.5), (14, 2.0))]
+    diagrams += [_cnf_diagram(12, 4.0, 5, inputs="0" * 12)]  # scalar result
+    diagrams += [_random_diagram(rng, int(rng.integers(2, 40)), int(rng.integers(4, 24)), int(rng.integers(0, 6)))
+                 for _ in range(25)]
+    # 2^10 terms in one step: counts of 0 mod 256
+    diagrams.append(Diagram(Wiring([2] * 12, [[*range(11)], [*range(10), 11]], [11, 10]),
+                            [np.ones((2,) * 11, np.uint8)] * 2))
+    with DeviceRel.mode_scope(mode):
+        for i, d in enumerate(diagrams):
+            c = PlannedContraction(DeviceRel, d.wiring)
+            print(f"{mode} diagram {i}: {d.wiring.num_slots} slots, {len(d.wiring.out_wires)} out", flush=True)
+            first, again = c.contract(d), c.contract(d)
+            assert c._small is not None
+            c._small = None  # the walk
+            walk = c.contract(d)
+            assert first.tensor_shape == walk.tensor_shape
+            np.testing.assert_array_equal(first.tensor, walk.tensor)
+            np.testing.assert_array_equal(again.tensor, walk.tensor)
+            if mode == "GT0":
+                np.testing.assert_array_equal(walk.tensor,
+                                              PlannedContraction(OracleRel, d.wiring).contract(d).tensor)
+
+
+@pytest.mark.gpu
+def test_device_blocks_and_other_streams():
+    import torch
+
+    from tensorsat_amd.rel import DeviceRel
+
+    d = _cnf_diagram(8, 3.0, 1)
+    c = PlannedContraction(DeviceRel, d.wiring)
+    want = c.contract(d).tensor
+    boxes = Diagram(d.wiring, [DeviceRel(np.asarray(b)) for b in d.blocks])
+    np.testing.assert_array_equal(c.contract(boxes).tensor, want)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        other = c.contract(d)
+    s.synchronize()
+    np.testing.assert_array_equal(other.tensor, want)
