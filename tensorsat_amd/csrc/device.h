@@ -22,6 +22,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include "../../include/tensorsat_amd.h"
@@ -43,6 +44,24 @@ using Lut = LutT<4>;
 
 __device__ __forceinline__ int nchunks(int bits) { return (bits + 7) >> 3; }
 
+// 8 bytes of a record from byte `off` on, from its aligned dwords.
+__device__ __forceinline__ uint64_t rec8(const uint32_t* w, size_t off) {
+  const int q = (int)(off >> 2), r = (int)(off & 3);
+  const uint64_t lo = (uint64_t)w[q] | ((uint64_t)w[q + 1] << 32);
+  return r == 0 ? lo : (lo >> (8 * r)) | ((uint64_t)w[q + 2] << (64 - 8 * r));
+}
+
+// The low n (<= 8) bits of v at the positions in pos (one byte each, TS_NOPOS: dropped).
+// TS_NOPOS shifts its bit to position 31, as do the bytes from the n-th on; positions are
+// below TS_MAX_BITS, so bit 31 is cleared at the end.
+__device__ __forceinline__ uint32_t place8(uint32_t v, int n, uint64_t pos) {
+  if (n < 8) pos |= ~0ull << (8 * n);
+  uint32_t off = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) off |= ((v >> i) & 1u) << ((uint32_t)(pos >> (8 * i)) & 31u);
+  return off & 0x7fffffffu;
+}
+
 // Build the chunk tables of one step (all threads of the workgroup participate; the
 // caller synchronises afterwards).
 template <int NQ>
@@ -52,20 +71,11 @@ __device__ inline void build_lut(const ts_step& st, LutT<NQ>& L, bool need_c, in
   // be 0 and not a value left in LDS by an earlier step.
   int nqo = nchunks(ro) > 0 ? nchunks(ro) : 1;
   nqo = nqo < NQ ? nqo : NQ;  // callers keep ranks within the table (16 bits for NQ = 2)
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(&st);
   for (int e = tid; e < nqo * 256; e += WG) {
-    const int q = e >> 8, v = e & 255;
-    uint32_t al = 0, ar = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int j = q * 8 + i;
-      if (j < ro && ((v >> i) & 1)) {
-        const uint8_t pl = st.o_lpos[j], pr = st.o_rpos[j];
-        if (pl != TS_NOPOS) al |= 1u << pl;
-        if (pr != TS_NOPOS) ar |= 1u << pr;
-      }
-    }
-    L.ol[q][v] = al;
-    L.orr[q][v] = ar;
+    const int q = e >> 8, left = ro - 8 * q, n = left < 0 ? 0 : left < 8 ? left : 8;
+    L.ol[q][e & 255] = place8((uint32_t)e & 255u, n, rec8(w + 2 * q, offsetof(ts_step, o_lpos)));
+    L.orr[q][e & 255] = place8((uint32_t)e & 255u, n, rec8(w + 2 * q, offsetof(ts_step, o_rpos)));
   }
   if (need_c) {
     const int nc = st.sum_rank;
@@ -153,149 +163,172 @@ __device__ __forceinline__ uint64_t load_row(const uint8_t* p, int nc) {
 
 // ---- vector path for short rows ------------------------------------------------------
 //
-// When, in each operand, the low t out bits it holds sit right above its summed bits in
-// order (the others not held at all), the rows of 2^t consecutive outputs lie in one
-// chunk of 2^(sum + held) bytes: a lane loads each operand's chunk once (at most 32
-// bytes), picks the row of each of its 2^t outputs out of it, and stores the 2^t results
-// at once.
+// Rows of 1..8 bytes (at most 3 summed bits, innermost).  Where each operand holds the two
+// lowest out bits right above its summed bits in order (or not at all) -- the compiler lays
+// out every operand so -- the rows of 4 consecutive outputs are one run of at most 32 bytes.
+// A lane computes 16 consecutive outputs as four such groups: out bits 2 and 3 just move the
+// run's address, so all its loads go out at once, and the rows are combined a dword at a
+// time (v_perm picks the four outputs' bytes of one term; rows of 4 and 8 bytes are whole
+// dwords).  Counts are at most 64, so both epilogues reduce to "any bit of the AND set".
+// Bound by HBM and, on many workgroups, by their tables: 16 jobs of 2^23 outputs on 65536
+// workgroups took 336 us with each output's row picked out of a chunk held in 64-bit words
+// (40 vector instructions per output), 288 us with dwords (6), and 75 us once 8192 workgroups
+// shared the work.
 
-// t (0 = no vector path, at most 4) and the held low out bits of each operand.
-__host__ __device__ inline int vec_plan(const ts_step& st, uint32_t& ml, uint32_t& mr) {
-  ml = mr = 0;
+__host__ __device__ inline bool quad_shaped(const ts_step& st) {
   const int nc = st.sum_rank;
-  if (nc > 3 || !(nc == 0 || (st.flags & TS_STEP_KINNER))) return 0;
+  if (nc > 3 || !(nc == 0 || (st.flags & TS_STEP_KINNER)) || st.out_rank < 4) return false;
   const bool norhs = st.flags & TS_STEP_NORHS;
-  const int tmax = st.out_rank < 4 ? st.out_rank : 4;
-  int best = 0, hl = 0, hr = 0;
-  uint32_t cl = 0, cr = 0;
-  for (int t = 1; t <= tmax; ++t) {
-    const int j = t - 1;
-    if (st.o_lpos[j] != TS_NOPOS) {
-      if (st.o_lpos[j] != nc + hl) break;
-      cl |= 1u << j;
-      ++hl;
-    }
-    if (!norhs && st.o_rpos[j] != TS_NOPOS) {
-      if (st.o_rpos[j] != nc + hr) break;
-      cr |= 1u << j;
-      ++hr;
-    }
-    if (nc + hl > 5 || nc + hr > 5) break;  // chunks of at most 32 bytes
-    best = t;
-    ml = cl;
-    mr = cr;
+  int hl = 0, hr = 0;
+  for (int j = 0; j < 2; ++j) {
+    if (st.o_lpos[j] != TS_NOPOS && st.o_lpos[j] != nc + hl++) return false;
+    if (!norhs && st.o_rpos[j] != TS_NOPOS && st.o_rpos[j] != nc + hr++) return false;
   }
-  return best;
+  return true;
 }
 
-// 2^lg bytes (lg <= 5) into 64-bit words.
-__device__ __forceinline__ void load_chunk(uint64_t (&w)[4], const uint8_t* p, int lg) {
-  switch (lg) {
-    case 0: w[0] = *p; break;
-    case 1: w[0] = *reinterpret_cast<const uint16_t*>(p); break;
-    case 2: w[0] = *reinterpret_cast<const uint32_t*>(p); break;
-    case 3: w[0] = *reinterpret_cast<const uint64_t*>(p); break;
-    case 4: {
-      const uint4 v = *reinterpret_cast<const uint4*>(p);
-      w[0] = ((uint64_t)v.y << 32) | v.x;
-      w[1] = ((uint64_t)v.w << 32) | v.z;
-      break;
-    }
-    default: {
-      const uint4 v = reinterpret_cast<const uint4*>(p)[0], u = reinterpret_cast<const uint4*>(p)[1];
-      w[0] = ((uint64_t)v.y << 32) | v.x;
-      w[1] = ((uint64_t)v.w << 32) | v.z;
-      w[2] = ((uint64_t)u.y << 32) | u.x;
-      w[3] = ((uint64_t)u.w << 32) | u.z;
-    }
-  }
-}
-
-// Row idx (2^K bytes) of a chunk held as 64-bit words (word picked by selects: no
-// indexed register access).
-template <int K>
-__device__ __forceinline__ uint64_t chunk_row(const uint64_t (&w)[4], uint32_t idx) {
-  const uint32_t off = idx << K, q = off >> 3;
-  const uint64_t word = q == 0 ? w[0] : q == 1 ? w[1] : q == 2 ? w[2] : w[3];
-  if constexpr (K == 3) {
-    return word;
+// 2^LG bytes (LG <= 5) as dwords.
+template <int LG>
+struct Run {
+  uint32_t w[LG < 4 ? 2 : 1 << (LG - 2)];
+};
+template <int LG>
+__device__ __forceinline__ Run<LG> load_run(const uint8_t* p) {
+  Run<LG> r;
+  if constexpr (LG <= 2) {
+    r.w[1] = 0;
+    if constexpr (LG == 0) r.w[0] = *p;
+    else if constexpr (LG == 1) r.w[0] = *reinterpret_cast<const uint16_t*>(p);
+    else r.w[0] = *reinterpret_cast<const uint32_t*>(p);
+  } else if constexpr (LG == 3) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    r.w[0] = v.x;
+    r.w[1] = v.y;
   } else {
-    constexpr uint64_t MASK = (1ull << (8 << K)) - 1;
-    return (word >> (8 * (off & 7))) & MASK;
-  }
-}
-
-// Bits of i (< 16) at the set positions of m, packed low.
-__device__ __forceinline__ uint32_t pext4(uint32_t i, uint32_t m) {
-  uint32_t r = 0, b = 0;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-    if ((m >> j) & 1u) r |= ((i >> j) & 1u) << b++;
+    for (int h = 0; h < (1 << (LG - 4)); ++h) {
+      const uint4 v = reinterpret_cast<const uint4*>(p)[h];
+      r.w[4 * h] = v.x;
+      r.w[4 * h + 1] = v.y;
+      r.w[4 * h + 2] = v.z;
+      r.w[4 * h + 3] = v.w;
+    }
+  }
   return r;
 }
 
-template <int K, int V, int NQ>
-__device__ void step_vec_kv(const ts_step& st, const LutT<NQ>& L, const uint8_t* __restrict__ lhs,
-                            const uint8_t* __restrict__ rhs, uint8_t* __restrict__ out, uint64_t first,
-                            uint64_t stride, uint32_t ml, uint32_t mr) {
-  constexpr int T = V == 2 ? 1 : V == 4 ? 2 : V == 8 ? 3 : 4;
+// Index of output i's row in an operand that holds H of the two lowest out bits (H = 1: bit
+// `one` of them).
+template <int H>
+__device__ __forceinline__ uint32_t quad_row(int i, int one) {
+  return H == 0 ? 0u : H == 2 ? (uint32_t)i : (uint32_t)(i >> one) & 1u;
+}
+
+// Byte c of the four outputs' rows (K <= 1).
+template <int K, int H>
+__device__ __forceinline__ uint32_t quad_bytes(const Run<K + H>& r, uint32_t sel, int c) {
+  return __builtin_amdgcn_perm(r.w[1], r.w[0], sel + 0x01010101u * (uint32_t)c);
+}
+
+// Dword d of output i's row (K >= 2).
+template <int K, int H>
+__device__ __forceinline__ uint32_t quad_word(const Run<K + H>& r, int i, int d, int one) {
+  constexpr int D = 1 << (K - 2);
+  if constexpr (H == 1) return one ? r.w[(i >> 1) * D + d] : r.w[(i & 1) * D + d];
+  else return r.w[(H == 0 ? 0 : i) * D + d];
+}
+
+template <int K, int HL, int HR, int NQ>
+__device__ void step_quad_kh(const ts_step& st, const LutT<NQ>& L, const uint8_t* __restrict__ lhs,
+                             const uint8_t* __restrict__ rhs, uint8_t* __restrict__ out, uint64_t first,
+                             uint64_t stride) {
   const bool norhs = st.flags & TS_STEP_NORHS;
-  const int lgl = K + __popc(ml), lgr = K + __popc(mr);
   const int nqo = nchunks(st.out_rank);
-  const uint64_t nq = 1ull << (st.out_rank - T);
-  if (first >= nq) return;
-  const uint32_t lo = (uint32_t)((first << T) & 255);  // the same for every q of this lane
+  const uint64_t n = 1ull << (st.out_rank - 4);
+  if (first >= n) return;
+  const int one_l = st.o_lpos[0] == TS_NOPOS, one_r = norhs || st.o_rpos[0] == TS_NOPOS;
+  uint32_t dl[2], dr[2];  // what out bits 2 and 3 add to the offsets
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    dl[j] = st.o_lpos[2 + j] != TS_NOPOS ? 1u << st.o_lpos[2 + j] : 0u;
+    dr[j] = !norhs && st.o_rpos[2 + j] != TS_NOPOS ? 1u << st.o_rpos[2 + j] : 0u;
+  }
+  uint32_t sl = 0, sr = 0;  // byte selectors of term 0 (K <= 1)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    sl |= (quad_row<HL>(i, one_l) << K) << (8 * i);
+    sr |= (quad_row<HR>(i, one_r) << K) << (8 * i);
+  }
+  const uint32_t lo = (uint32_t)((first << 4) & 255);  // the same for every trip of this lane
   const uint32_t lo_l = L.ol[0][lo], lo_r = L.orr[0][lo];
-  for (uint64_t q = first; q < nq; q += stride) {
-    const uint64_t o = q << T;
+  for (uint64_t q = first; q < n; q += stride) {
+    const uint64_t o = q << 4;
     const uint32_t hi = (uint32_t)(o >> 8);
-    uint64_t a[4] = {0, 0, 0, 0}, b[4] = {0, 0, 0, 0};
-    load_chunk(a, lhs + lo_l + hi_off<NQ>(L.ol, hi, nqo), lgl);
-    if (!norhs) load_chunk(b, rhs + lo_r + hi_off<NQ>(L.orr, hi, nqo), lgr);
-    uint32_t res[(V + 3) / 4];
+    const uint8_t* pl = lhs + lo_l + hi_off<NQ>(L.ol, hi, nqo);
+    const uint8_t* pr = rhs + lo_r + hi_off<NQ>(L.orr, hi, nqo);
+    Run<K + HL> a[4];
+    Run<K + HR> b[4];
 #pragma unroll
-    for (int i = 0; i < (V + 3) / 4; ++i) res[i] = 0;
+    for (int g = 0; g < 4; ++g) a[g] = load_run<K + HL>(pl + ((g & 1 ? dl[0] : 0u) + (g & 2 ? dl[1] : 0u)));
+    if (!norhs) {
 #pragma unroll
-    for (int i = 0; i < V; ++i) {
-      uint64_t x = chunk_row<K>(a, pext4((uint32_t)i, ml));
-      if (!norhs) x &= chunk_row<K>(b, pext4((uint32_t)i, mr));
-      res[i / 4] |= (uint32_t)(x != 0) << (8 * (i % 4));
+      for (int g = 0; g < 4; ++g) b[g] = load_run<K + HR>(pr + ((g & 1 ? dr[0] : 0u) + (g & 2 ? dr[1] : 0u)));
+    } else {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (uint32_t& w : b[g].w) w = ~0u;
     }
-    uint8_t* po = out + o;
-    if constexpr (V == 16) *reinterpret_cast<uint4*>(po) = make_uint4(res[0], res[1], res[2], res[3]);
-    else if constexpr (V == 8) *reinterpret_cast<uint2*>(po) = make_uint2(res[0], res[1]);
-    else if constexpr (V == 4) *reinterpret_cast<uint32_t*>(po) = res[0];
-    else *reinterpret_cast<uint16_t*>(po) = (uint16_t)res[0];
+    uint32_t res[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      if constexpr (K <= 1) {
+        uint32_t x = quad_bytes<K, HL>(a[g], sl, 0) & quad_bytes<K, HR>(b[g], sr, 0);
+        if constexpr (K == 1) x |= quad_bytes<K, HL>(a[g], sl, 1) & quad_bytes<K, HR>(b[g], sr, 1);
+        res[g] = ((((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x) >> 7) & 0x01010101u;
+      } else {
+        res[g] = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          uint32_t x = quad_word<K, HL>(a[g], i, 0, one_l) & quad_word<K, HR>(b[g], i, 0, one_r);
+          if constexpr (K == 3) x |= quad_word<K, HL>(a[g], i, 1, one_l) & quad_word<K, HR>(b[g], i, 1, one_r);
+          res[g] |= (x < 1u ? x : 1u) << (8 * i);
+        }
+      }
+    }
+    *reinterpret_cast<uint4*>(out + o) = make_uint4(res[0], res[1], res[2], res[3]);
   }
 }
 
-// Grid-stride over groups of 2^t outputs, t = vec_plan(st, ml, mr) (first / stride as
-// for step_u8).  Counts are at most 8, so both epilogues reduce to count != 0.
+template <int K, int HL, int NQ>
+__device__ __forceinline__ void step_quad_k(const ts_step& st, int hr, const LutT<NQ>& L, const uint8_t* lhs,
+                                            const uint8_t* rhs, uint8_t* out, uint64_t first, uint64_t stride) {
+  if (hr == 0) step_quad_kh<K, HL, 0, NQ>(st, L, lhs, rhs, out, first, stride);
+  else if (hr == 1) step_quad_kh<K, HL, 1, NQ>(st, L, lhs, rhs, out, first, stride);
+  else step_quad_kh<K, HL, 2, NQ>(st, L, lhs, rhs, out, first, stride);
+}
+
+template <int K, int NQ>
+__device__ __forceinline__ void step_quad_l(const ts_step& st, int hl, int hr, const LutT<NQ>& L, const uint8_t* lhs,
+                                            const uint8_t* rhs, uint8_t* out, uint64_t first, uint64_t stride) {
+  if (hl == 0) step_quad_k<K, 0, NQ>(st, hr, L, lhs, rhs, out, first, stride);
+  else if (hl == 1) step_quad_k<K, 1, NQ>(st, hr, L, lhs, rhs, out, first, stride);
+  else step_quad_k<K, 2, NQ>(st, hr, L, lhs, rhs, out, first, stride);
+}
+
+// Grid-stride over groups of 16 outputs of a quad_shaped step (first / stride as for
+// step_u8).
 template <int NQ>
-__device__ void step_u8_vec(const ts_step& st, const LutT<NQ>& L, const uint8_t* __restrict__ lhs,
-                            const uint8_t* __restrict__ rhs, uint8_t* __restrict__ out, uint64_t first,
-                            uint64_t stride, int t, uint32_t ml, uint32_t mr) {
-#define TS_VEC(K, V) step_vec_kv<K, V, NQ>(st, L, lhs, rhs, out, first, stride, ml, mr)
-  switch (st.sum_rank * 8 + t) {
-    case 0 * 8 + 1: TS_VEC(0, 2); break;
-    case 0 * 8 + 2: TS_VEC(0, 4); break;
-    case 0 * 8 + 3: TS_VEC(0, 8); break;
-    case 0 * 8 + 4: TS_VEC(0, 16); break;
-    case 1 * 8 + 1: TS_VEC(1, 2); break;
-    case 1 * 8 + 2: TS_VEC(1, 4); break;
-    case 1 * 8 + 3: TS_VEC(1, 8); break;
-    case 1 * 8 + 4: TS_VEC(1, 16); break;
-    case 2 * 8 + 1: TS_VEC(2, 2); break;
-    case 2 * 8 + 2: TS_VEC(2, 4); break;
-    case 2 * 8 + 3: TS_VEC(2, 8); break;
-    case 2 * 8 + 4: TS_VEC(2, 16); break;
-    case 3 * 8 + 1: TS_VEC(3, 2); break;
-    case 3 * 8 + 2: TS_VEC(3, 4); break;
-    case 3 * 8 + 3: TS_VEC(3, 8); break;
-    case 3 * 8 + 4: TS_VEC(3, 16); break;
-    default: break;
-  }
-#undef TS_VEC
+__device__ inline void step_quad(const ts_step& st, const LutT<NQ>& L, const uint8_t* __restrict__ lhs,
+                                 const uint8_t* __restrict__ rhs, uint8_t* __restrict__ out, uint64_t first,
+                                 uint64_t stride) {
+  const bool norhs = st.flags & TS_STEP_NORHS;
+  const int hl = (st.o_lpos[0] != TS_NOPOS) + (st.o_lpos[1] != TS_NOPOS);
+  const int hr = norhs ? 0 : (st.o_rpos[0] != TS_NOPOS) + (st.o_rpos[1] != TS_NOPOS);
+  if (st.sum_rank == 0) step_quad_l<0, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
+  else if (st.sum_rank == 1) step_quad_l<1, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
+  else if (st.sum_rank == 2) step_quad_l<2, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
+  else step_quad_l<3, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
 }
 
 // Boolean step over out indices o = first + k * stride (first = block * 256 + tid and

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstddef>
 #include <cstring>
 #include <vector>
 
@@ -37,10 +38,8 @@ __global__ __launch_bounds__(WG) void k_step_u8(const uint8_t* __restrict__ lhs,
   const bool need_c = !(st.flags & TS_STEP_KINNER) && st.sum_rank > 0;
   build_lut(st, L, need_c, threadIdx.x);
   __syncthreads();
-  uint32_t ml, mr;
-  const int t = vec_plan(st, ml, mr);
-  if (t > 0)
-    step_u8_vec(st, L, lhs, rhs, out, (uint64_t)blockIdx.x * WG + threadIdx.x, (uint64_t)gridDim.x * WG, t, ml, mr);
+  if (quad_shaped(st))
+    step_quad(st, L, lhs, rhs, out, (uint64_t)blockIdx.x * WG + threadIdx.x, (uint64_t)gridDim.x * WG);
   else
     step_u8(st, L, lhs, rhs, out, (uint64_t)blockIdx.x * WG + threadIdx.x, (uint64_t)gridDim.x * WG, mode);
 }
@@ -277,12 +276,11 @@ __device__ void seq_run(uint8_t* __restrict__ arena, const ts_step* __restrict__
     const uint8_t* rhs = arena + (norhs ? st.lhs_off : st.rhs_off);
     if (ro <= 8 && (kinner || nc == 0)) {
       if (tid < (1 << ro)) {
-        uint32_t offl = 0, offr = 0;
-        for (int j = 0; j < ro; ++j)
-          if ((tid >> j) & 1) {
-            if (st.o_lpos[j] != TS_NOPOS) offl |= 1u << st.o_lpos[j];
-            if (st.o_rpos[j] != TS_NOPOS) offr |= 1u << st.o_rpos[j];
-          }
+        // Both position lists as a few dwords of the record, read together and decoded in
+        // registers: reading them byte by byte under each bit's test was most of a step.
+        const uint32_t* w = reinterpret_cast<const uint32_t*>(&st);
+        const uint32_t offl = place8((uint32_t)tid, ro, rec8(w, offsetof(ts_step, o_lpos)));
+        const uint32_t offr = place8((uint32_t)tid, ro, rec8(w, offsetof(ts_step, o_rpos)));
         uint32_t acc;
         if (nc == 0) {
           acc = lhs[offl];
@@ -311,7 +309,7 @@ __global__ __launch_bounds__(WG) void k_step_seq(uint8_t* __restrict__ arena, co
 // A whole small job in one launch: the leaves come as bits in the kernel arguments, the arena
 // is in LDS, and only the result goes to memory.  Bound by the chain of steps (about half a
 // microsecond each); a launch per step costs 3 us of the device and ten times that of the
-// host.  158 steps, result of 2^10 entries: 5.9 ms as uploads and launches per step, 143
+// host.  158 steps, result of 2^10 entries: 5.9 ms as uploads and launches per step, 97
 // us so.
 constexpr int LEAF_WORDS = 896;  // 28672 leaf entries; the arguments stay below 4 KiB
 struct SmallJob {
@@ -337,6 +335,10 @@ __global__ __launch_bounds__(WG) void k_small_job(SmallJob) {
 // value (kernarg above).
 
 constexpr int GANG = 64;
+// Blocks of one launch of large steps.  Each builds its step's tables first (a few us), so
+// they are few and long: 16 jobs of 2^23 outputs take 288 us on 65536 blocks of half a trip
+// each, 75 us on 8192 of four.
+constexpr uint64_t STEP_CAP = 8192;
 
 struct GangSeq {  // one workgroup per job: a run of small steps
   const ts_step* steps[GANG];
@@ -393,9 +395,10 @@ __global__ __launch_bounds__(WG) void k_gang_step(GangStep) {
   __shared__ uint32_t part[WG / 64];
   const GangStep& g = kernarg<GangStep>();
   const uint32_t b = blockIdx.x;
-  int j = 0;
-  while (j + 1 < g.n && g.blk[j + 1] <= b) ++j;
   const int tid = threadIdx.x;
+  // The job of this block: jobs before it end at or below it (one load per lane).
+  const int at = tid & 63;
+  const int j = __popcll(__ballot(at + 1 < g.n && g.blk[at + 1] <= b));
   if (tid < (int)(sizeof(ts_step) / 16))
     reinterpret_cast<uint4*>(&s_st)[tid] = reinterpret_cast<const uint4*>(g.rec[j])[tid];
   __syncthreads();
@@ -428,11 +431,8 @@ __global__ __launch_bounds__(WG) void k_gang_step(GangStep) {
   }
   build_lut(s_st, L, !kinner && s_st.sum_rank > 0, tid);
   __syncthreads();
-  uint32_t ml, mr;
-  const int t = vec_plan(s_st, ml, mr);
-  if (t > 0)
-    step_u8_vec(s_st, L, arena + s_st.lhs_off, rhs, arena + s_st.out_off, (uint64_t)first * WG + tid,
-                (uint64_t)nb * WG, t, ml, mr);
+  if (quad_shaped(s_st))
+    step_quad(s_st, L, arena + s_st.lhs_off, rhs, arena + s_st.out_off, (uint64_t)first * WG + tid, (uint64_t)nb * WG);
   else
     step_u8(s_st, L, arena + s_st.lhs_off, rhs, arena + s_st.out_off, (uint64_t)first * WG + tid, (uint64_t)nb * WG,
             g.mode);
@@ -1002,6 +1002,15 @@ int make_step(int rl, const int32_t* lw, int rr, const int32_t* rw, int ro, cons
   return TS_OK;
 }
 
+// Workgroups of one step on the step engine.  Short rows (quad_shaped) take 4096 outputs per
+// trip, and a workgroup's tables cost as much as a few trips, so at most 2048 of them (8 per
+// CU); other steps take 256 outputs or more per trip.
+uint64_t step_blocks(const ts_step& st) {
+  const uint64_t n = 1ull << st.out_rank;
+  if (quad_shaped(st)) return std::min<uint64_t>((n + 16 * WG - 1) / (16 * WG), 2048);
+  return (uint64_t)grid_for(n);
+}
+
 int launch_step_u8(const uint8_t* lhs, const uint8_t* rhs, uint8_t* out, const ts_step& st, int mode,
                    hipStream_t s) {
   if (tsd::dense_eligible(st, lhs, rhs)) return tsd::launch_dense(lhs, rhs, out, st, mode, s);
@@ -1009,7 +1018,7 @@ int launch_step_u8(const uint8_t* lhs, const uint8_t* rhs, uint8_t* out, const t
     hipLaunchKernelGGL(k_step_dot, dim3(1u << st.out_rank), dim3(WG), 0, s, lhs, rhs, out, st, mode);
     return hip_rc(hipGetLastError());
   }
-  hipLaunchKernelGGL(k_step_u8, dim3(grid_for(1ull << st.out_rank)), dim3(WG), 0, s, lhs, rhs, out, st, mode);
+  hipLaunchKernelGGL(k_step_u8, dim3((uint32_t)step_blocks(st)), dim3(WG), 0, s, lhs, rhs, out, st, mode);
   return hip_rc(hipGetLastError());
 }
 
@@ -1131,14 +1140,13 @@ ContractPlan plan_contract(const ts_step& s0, bool aligned) {
     if (kinner) return p;
     p.kind = PLAN_DENSE;
   } else if (nc <= 7 && st.out_rank >= OUT_MIN) {
-    uint32_t ml, mr;
     auto rows_in_order = [&](const uint8_t* pos) {  // kept bits right above the summed ones
       int k = nc;
       for (int j = 0; j < st.out_rank && k < 6; ++j)
         if (pos[j] != TS_NOPOS && pos[j] != k++) return false;
       return true;
     };
-    if (kinner && vec_plan(st, ml, mr) == 4 && rows_in_order(st.o_lpos) && rows_in_order(st.o_rpos)) return p;
+    if (kinner && quad_shaped(st) && rows_in_order(st.o_lpos) && rows_in_order(st.o_rpos)) return p;
     p.kind = PLAN_OUTER;
   } else {
     if (kinner || st.out_rank + nc < TERM_MIN) return p;
@@ -1761,9 +1769,9 @@ int ts_program_run_gang(const ts_job* jobs, int32_t count, const ts_step* steps,
       if (!nt) return TS_OK;
       const int prc = flush_pack();
       if (prc) return prc;
-      // at most 65536 blocks per launch, every job keeping at least one (grid-stride
+      // at most STEP_CAP blocks per launch, every job keeping at least one (grid-stride
       // loops take any count); one-block-per-output jobs keep theirs
-      const uint64_t cap = 65536;
+      const uint64_t cap = STEP_CAP;
       uint32_t at = 0;
       for (int k = 0; k < nt; ++k) {
         t.blk[k] = at;
@@ -1823,7 +1831,7 @@ int ts_program_run_gang(const ts_job* jobs, int32_t count, const ts_step* steps,
         t.kind[nt] = 2;
         t.pk[nt] = (uint32_t)pk;
       }
-      const uint64_t b = t.kind[nt] == 1 ? (1ull << st.out_rank) : (uint64_t)grid_for(1ull << st.out_rank);
+      const uint64_t b = t.kind[nt] == 1 ? (1ull << st.out_rank) : step_blocks(st);
       wants.push_back(b);
       if (t.kind[nt] != 1) want += b;
       if (++nt == GANG) {
