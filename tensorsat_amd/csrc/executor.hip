@@ -396,9 +396,12 @@ __global__ __launch_bounds__(WG) void k_gang_step(GangStep) {
   const GangStep& g = kernarg<GangStep>();
   const uint32_t b = blockIdx.x;
   const int tid = threadIdx.x;
-  // The job of this block: jobs before it end at or below it (one load per lane).
-  const int at = tid & 63;
-  const int j = __popcll(__ballot(at + 1 < g.n && g.blk[at + 1] <= b));
+  // The job of this block: the last one that starts at or below it, by halving.  Scalar loads
+  // only: a wave-wide ballot here went wrong where one lane alone uses the job (below: it took
+  // another job's mask offset).
+  int j = 0;
+  for (int h = GANG / 2; h > 0; h >>= 1)
+    if (j + h < g.n && g.blk[j + h] <= b) j += h;
   if (tid < (int)(sizeof(ts_step) / 16))
     reinterpret_cast<uint4*>(&s_st)[tid] = reinterpret_cast<const uint4*>(g.rec[j])[tid];
   __syncthreads();

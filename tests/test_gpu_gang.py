@@ -119,3 +119,48 @@ def test_gang_packed_rows(seed, k):
             want = run_job_fused(dp, g, mode).cpu().numpy()
             np.testing.assert_array_equal(got, want, err_msg=f"slice {g} {mode}")
             assert flags[g] == int(want.any())
+
+
+def _first_packed_step(prog, j):
+    """Index in job j of its first step whose rows gang execution packs, or None."""
+    b, n = int(prog.jobs["step_begin"][j]), int(prog.jobs["num_steps"][j])
+    for i, st in enumerate(prog.steps[b : b + n]):
+        ro, k = int(st["out_rank"]), int(st["sum_rank"])
+        held = (st["o_lpos"][:ro] != PG.NOPOS) != (st["o_rpos"][:ro] != PG.NOPOS)
+        if (st["flags"] & 3) == PG.STEP_KINNER and 4 <= k <= 5 and ro >= 12 and held.sum() >= 2:
+            return i
+    return None
+
+
+def test_gang_packed_rows_of_different_jobs():
+    """Jobs of different arena sizes whose packed steps run in one launch: each job's masks are
+    its own.  The gang runs every job up to its first packed step, whose whole output is
+    compared with the one-step-at-a-time runner's."""
+    import torch
+
+    from tensorsat_amd.executor import DeviceProgram, gang_stride, run_gang, run_job
+
+    progs, rng = [], np.random.default_rng(4)
+    while len(progs) < 6:
+        cnf = CNFInstance.random(3, 110, 440, rng=int(rng.integers(1 << 30)))
+        p = PG.sat_batch([cnf], width=24, max_cubes=1)
+        if len(p.jobs) == 1 and _first_packed_step(p, 0) is not None:
+            progs.append(p)
+    prog = PG.concat(progs, [np.array([i]) for i in range(6)], 6)
+    assert len(set(prog.jobs["arena_elems"].tolist())) > 1
+    dp = DeviceProgram(prog)
+    stride = gang_stride(dp)
+    last = [_first_packed_step(prog, j) for j in range(6)]
+    want = [run_job(dp, j, "GT0", keep_intermediates=True)[1][last[j]] for j in range(6)]
+    for j in range(6):
+        dp.jobs_host["num_steps"][j] = last[j] + 1
+        dp.jobs_host["result_off"][j] = prog.steps["out_off"][prog.jobs["step_begin"][j] + last[j]]
+        dp.jobs_host["result_rank"][j] = prog.steps["out_rank"][prog.jobs["step_begin"][j] + last[j]]
+    for mode in ("GT0", "MOD256"):
+        for small_bits in (12, 0):
+            arena = torch.full((6 * stride,), 255, dtype=torch.uint8, device="cuda")
+            run_gang(dp, 0, 6, mode, arena=arena, small_bits=small_bits)
+            for j in range(6):
+                o, n = j * stride + int(dp.jobs_host["result_off"][j]), 1 << int(dp.jobs_host["result_rank"][j])
+                print(f"{mode} small {small_bits} job {j}: step {last[j]}, {n} outputs", flush=True)
+                assert torch.equal(arena[o : o + n], want[j])
