@@ -12,7 +12,13 @@ namespace tsd {
 // the MFMA route is enabled (ts_dense_config).
 bool dense_eligible(const ts_step& st, const void* lhs, const void* rhs);
 
-int launch_dense(const uint8_t* lhs, const uint8_t* rhs, uint8_t* out, const ts_step& st, int mode,
-                 hipStream_t s);
+constexpr int DENSE_GANG = 64;  // jobs of one launch
+
+// True when two records differ at most in their operands' offsets.
+bool same_dense_step(const ts_step& x, const ts_step& y);
+
+// The step on n (1..DENSE_GANG) sets of operands in one launch.
+int launch_dense(int n, const uint8_t* const* lhs, const uint8_t* const* rhs, uint8_t* const* out, const ts_step& st,
+                 int mode, hipStream_t s);
 
 }  // namespace tsd

@@ -44,21 +44,21 @@ using Lut = LutT<4>;
 
 __device__ __forceinline__ int nchunks(int bits) { return (bits + 7) >> 3; }
 
-// 8 bytes of a record from byte `off` on, from its aligned dwords.
-__device__ __forceinline__ uint64_t rec8(const uint32_t* w, size_t off) {
+// 8 bytes of a record from byte `off` on (a constant), from its aligned dwords.
+__device__ __forceinline__ uint2 rec8(const uint32_t* w, size_t off) {
   const int q = (int)(off >> 2), r = (int)(off & 3);
-  const uint64_t lo = (uint64_t)w[q] | ((uint64_t)w[q + 1] << 32);
-  return r == 0 ? lo : (lo >> (8 * r)) | ((uint64_t)w[q + 2] << (64 - 8 * r));
+  if (r == 0) return make_uint2(w[q], w[q + 1]);
+  return make_uint2(__builtin_amdgcn_alignbyte(w[q + 1], w[q], r), __builtin_amdgcn_alignbyte(w[q + 2], w[q + 1], r));
 }
 
-// The low n (<= 8) bits of v at the positions in pos (one byte each, TS_NOPOS: dropped).
-// TS_NOPOS shifts its bit to position 31, as do the bytes from the n-th on; positions are
-// below TS_MAX_BITS, so bit 31 is cleared at the end.
-__device__ __forceinline__ uint32_t place8(uint32_t v, int n, uint64_t pos) {
-  if (n < 8) pos |= ~0ull << (8 * n);
+// The low 8 bits of v at the positions in pos (one byte each); set bits of v beyond the ones
+// that exist are the caller's to clear.  TS_NOPOS shifts its bit to position 31; positions
+// are below TS_MAX_BITS, so bit 31 is cleared at the end.  Three 32-bit instructions per bit
+// (64-bit shifts of the position list were most of a small step).
+__device__ __forceinline__ uint32_t place8(uint32_t v, uint2 pos) {
   uint32_t off = 0;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) off |= ((v >> i) & 1u) << ((uint32_t)(pos >> (8 * i)) & 31u);
+  for (int i = 0; i < 8; ++i) off |= ((v >> i) & 1u) << (((i < 4 ? pos.x : pos.y) >> (8 * (i & 3))) & 31u);
   return off & 0x7fffffffu;
 }
 
@@ -73,9 +73,10 @@ __device__ inline void build_lut(const ts_step& st, LutT<NQ>& L, bool need_c, in
   nqo = nqo < NQ ? nqo : NQ;  // callers keep ranks within the table (16 bits for NQ = 2)
   const uint32_t* w = reinterpret_cast<const uint32_t*>(&st);
   for (int e = tid; e < nqo * 256; e += WG) {
-    const int q = e >> 8, left = ro - 8 * q, n = left < 0 ? 0 : left < 8 ? left : 8;
-    L.ol[q][e & 255] = place8((uint32_t)e & 255u, n, rec8(w + 2 * q, offsetof(ts_step, o_lpos)));
-    L.orr[q][e & 255] = place8((uint32_t)e & 255u, n, rec8(w + 2 * q, offsetof(ts_step, o_rpos)));
+    const int q = e >> 8, left = ro - 8 * q;
+    const uint32_t v = (uint32_t)e & (left < 8 ? (1u << left) - 1u : 255u);  // left >= 0
+    L.ol[q][e & 255] = place8(v, rec8(w + 2 * q, offsetof(ts_step, o_lpos)));
+    L.orr[q][e & 255] = place8(v, rec8(w + 2 * q, offsetof(ts_step, o_rpos)));
   }
   if (need_c) {
     const int nc = st.sum_rank;

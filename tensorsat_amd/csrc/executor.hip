@@ -279,8 +279,8 @@ __device__ void seq_run(uint8_t* __restrict__ arena, const ts_step* __restrict__
         // Both position lists as a few dwords of the record, read together and decoded in
         // registers: reading them byte by byte under each bit's test was most of a step.
         const uint32_t* w = reinterpret_cast<const uint32_t*>(&st);
-        const uint32_t offl = place8((uint32_t)tid, ro, rec8(w, offsetof(ts_step, o_lpos)));
-        const uint32_t offr = place8((uint32_t)tid, ro, rec8(w, offsetof(ts_step, o_rpos)));
+        const uint32_t offl = place8((uint32_t)tid, rec8(w, offsetof(ts_step, o_lpos)));
+        const uint32_t offr = place8((uint32_t)tid, rec8(w, offsetof(ts_step, o_rpos)));
         uint32_t acc;
         if (nc == 0) {
           acc = lhs[offl];
@@ -309,7 +309,7 @@ __global__ __launch_bounds__(WG) void k_step_seq(uint8_t* __restrict__ arena, co
 // A whole small job in one launch: the leaves come as bits in the kernel arguments, the arena
 // is in LDS, and only the result goes to memory.  Bound by the chain of steps (about half a
 // microsecond each); a launch per step costs 3 us of the device and ten times that of the
-// host.  158 steps, result of 2^10 entries: 5.9 ms as uploads and launches per step, 97
+// host.  158 steps, result of 2^10 entries: 5.9 ms as uploads and launches per step, 92
 // us so.
 constexpr int LEAF_WORDS = 896;  // 28672 leaf entries; the arguments stay below 4 KiB
 struct SmallJob {
@@ -340,10 +340,14 @@ constexpr int GANG = 64;
 // each, 75 us on 8192 of four.
 constexpr uint64_t STEP_CAP = 8192;
 
-struct GangSeq {  // one workgroup per job: a run of small steps
+// One workgroup per job: a run of small steps.  lds[j]: the run's tensors all lie in the first
+// lds[j] bytes of the job's arena, which are staged in LDS for the run and written back (0:
+// run in place).
+struct GangSeq {
   const ts_step* steps[GANG];
   uint8_t* arena[GANG];
   int32_t count[GANG];
+  int32_t lds[GANG];
   int32_t mode;
 };
 
@@ -381,12 +385,30 @@ struct GangAny {
   uint8_t* out;
 };
 
+// A step in device memory waits for its operands and for its stores to reach L2; in LDS it
+// waits less, so runs long enough to pay for moving their part of the arena there and
+// back are staged (SEQ_STAGE): 16 jobs of 631 steps on the first 15 KB 440 us in place, 400
+// us staged.
+constexpr int64_t SEQ_LDS = 65536;
+inline bool seq_staged(int steps, int64_t end) { return end <= SEQ_LDS && steps >= 8 && end <= 1024ll * steps; }
+
 __global__ __launch_bounds__(WG) void k_gang_seq(GangSeq) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t seq_arena[];
   __shared__ Lut L;
   __shared__ ts_step s_st[2];
   const GangSeq& g = kernarg<GangSeq>();
   const int j = blockIdx.x;
-  seq_run(g.arena[j], g.steps[j], g.count[j], g.mode, L, s_st);
+  uint8_t* arena = g.arena[j];
+  const int n16 = g.lds[j] >> 4;
+  if (n16 == 0) {
+    seq_run(arena, g.steps[j], g.count[j], g.mode, L, s_st);
+    return;
+  }
+  for (int i = threadIdx.x; i < n16; i += WG)
+    reinterpret_cast<uint4*>(seq_arena)[i] = reinterpret_cast<const uint4*>(arena)[i];
+  seq_run(seq_arena, g.steps[j], g.count[j], g.mode, L, s_st);  // starts and ends with a barrier
+  for (int i = threadIdx.x; i < n16; i += WG)
+    reinterpret_cast<uint4*>(arena)[i] = reinterpret_cast<const uint4*>(seq_arena)[i];
 }
 
 __global__ __launch_bounds__(WG) void k_gang_step(GangStep) {
@@ -1016,7 +1038,7 @@ uint64_t step_blocks(const ts_step& st) {
 
 int launch_step_u8(const uint8_t* lhs, const uint8_t* rhs, uint8_t* out, const ts_step& st, int mode,
                    hipStream_t s) {
-  if (tsd::dense_eligible(st, lhs, rhs)) return tsd::launch_dense(lhs, rhs, out, st, mode, s);
+  if (tsd::dense_eligible(st, lhs, rhs)) return tsd::launch_dense(1, &lhs, &rhs, &out, st, mode, s);
   if (dot_shaped(st)) {
     hipLaunchKernelGGL(k_step_dot, dim3(1u << st.out_rank), dim3(WG), 0, s, lhs, rhs, out, st, mode);
     return hip_rc(hipGetLastError());
@@ -1688,6 +1710,7 @@ int ts_program_run_gang(const ts_job* jobs, int32_t count, const ts_step* steps,
   // Segments per job: [begin, end) runs of small steps (kind 0) or one large step (kind 1).
   struct Seg {
     int begin, end, kind;
+    int64_t top;  // end of the arena bytes a run of small steps uses
   };
   std::vector<std::vector<Seg>> segs(count);
   size_t phases = 0;
@@ -1700,22 +1723,23 @@ int ts_program_run_gang(const ts_job* jobs, int32_t count, const ts_step* steps,
         job.result_off + (1ll << job.result_rank) > job.arena_elems)
       return TS_EINVAL;
     const ts_step* rec = steps + job.step_begin;
-    for (int i = 0; i < job.num_steps; ++i) {
-      const ts_step& st = rec[i];
-      const uint64_t hi = std::max<uint64_t>({st.lhs_off + (1ull << st.lhs_rank),
-                                               (st.flags & TS_STEP_NORHS) ? 0 : st.rhs_off + (1ull << st.rhs_rank),
-                                               st.out_off + (1ull << st.out_rank)});
-      if (hi > (uint64_t)job.arena_elems) return TS_EINVAL;
-    }
+    auto top = [](const ts_step& st) {
+      return (int64_t)std::max<uint64_t>({st.lhs_off + (1ull << st.lhs_rank),
+                                          (st.flags & TS_STEP_NORHS) ? 0 : st.rhs_off + (1ull << st.rhs_rank),
+                                          st.out_off + (1ull << st.out_rank)});
+    };
+    for (int i = 0; i < job.num_steps; ++i)
+      if (top(rec[i]) > job.arena_elems) return TS_EINVAL;
     int i = 0;
     while (i < job.num_steps) {
       if (small(rec[i])) {
-        int k = i + 1;
-        while (k < job.num_steps && small(rec[k])) ++k;
-        segs[g].push_back({i, k, 0});
+        int k = i;
+        int64_t end = 0;
+        for (; k < job.num_steps && small(rec[k]); ++k) end = std::max(end, top(rec[k]));
+        segs[g].push_back({i, k, 0, end});
         i = k;
       } else {
-        segs[g].push_back({i, i + 1, 1});
+        segs[g].push_back({i, i + 1, 1, 0});
         ++i;
       }
     }
@@ -1743,15 +1767,26 @@ int ts_program_run_gang(const ts_job* jobs, int32_t count, const ts_step* steps,
   for (size_t p = 0; p < phases; ++p) {
     // runs of small steps: one workgroup per job
     GangSeq q;
-    int nq = 0;
+    int nq = 0, seq_lds = 0;
     auto flush_seq = [&]() {
       if (!nq) return TS_OK;
       q.mode = mode;
-      hipLaunchKernelGGL(k_gang_seq, dim3(nq), dim3(WG), 0, s, q);
-      nq = 0;
+      hipLaunchKernelGGL(k_gang_seq, dim3(nq), dim3(WG), seq_lds, s, q);
+      nq = seq_lds = 0;
       return hip_rc(hipGetLastError());
     };
-    // large steps: MFMA-routed ones alone, the others shared out by block ranges
+    // MFMA-routed large steps: those of the same shape together
+    const uint8_t *dl[tsd::DENSE_GANG], *dr[tsd::DENSE_GANG];
+    uint8_t* dout[tsd::DENSE_GANG];
+    const ts_step* dst = nullptr;
+    int nd = 0;
+    auto flush_dense = [&]() {
+      if (!nd) return TS_OK;
+      const int drc = tsd::launch_dense(nd, dl, dr, dout, *dst, mode, s);
+      nd = 0;
+      return drc;
+    };
+    // the other large steps, shared out by block ranges
     GangStep t;
     int nt = 0;
     uint64_t want = 0;
@@ -1801,6 +1836,9 @@ int ts_program_run_gang(const ts_job* jobs, int32_t count, const ts_step* steps,
         q.steps[nq] = rec_dev + sg.begin;
         q.arena[nq] = ar;
         q.count[nq] = sg.end - sg.begin;
+        // whole 16-byte pieces: the stride is a multiple of 256, so they stay in this job's arena
+        q.lds[nq] = seq_staged(sg.end - sg.begin, sg.top) ? (int32_t)((sg.top + 15) & ~15ll) : 0;
+        seq_lds = std::max(seq_lds, q.lds[nq]);
         if (++nq == GANG) {
           const int rc = flush_seq();
           if (rc) return rc;
@@ -1811,8 +1849,14 @@ int ts_program_run_gang(const ts_job* jobs, int32_t count, const ts_step* steps,
       const uint8_t* lhs = ar + st.lhs_off;
       const uint8_t* rhs = ar + ((st.flags & TS_STEP_NORHS) ? st.lhs_off : st.rhs_off);
       if (tsd::dense_eligible(st, lhs, rhs)) {
-        const int rc = tsd::launch_dense(lhs, rhs, ar + st.out_off, st, mode, s);
-        if (rc) return rc;
+        if (nd && (nd == tsd::DENSE_GANG || !tsd::same_dense_step(st, *dst))) {
+          const int rc = flush_dense();
+          if (rc) return rc;
+        }
+        dst = &st;
+        dl[nd] = lhs;
+        dr[nd] = rhs;
+        dout[nd++] = ar + st.out_off;
         continue;
       }
       t.rec[nt] = rec_dev + sg.begin;
@@ -1843,6 +1887,8 @@ int ts_program_run_gang(const ts_job* jobs, int32_t count, const ts_step* steps,
       }
     }
     int rc = flush_seq();
+    if (rc) return rc;
+    rc = flush_dense();
     if (rc) return rc;
     rc = flush_step();
     if (rc) return rc;

@@ -73,6 +73,10 @@ def test_small_trees_match_the_walk_and_the_oracle(mode):
     # 2^10 terms in one step: counts of 0 mod 256
     diagrams.append(Diagram(Wiring([2] * 12, [[*range(11)], [*range(10), 11]], [11, 10]),
                             [np.ones((2,) * 11, np.uint8)] * 2))
+    # 16384 leaf entries and a result of 2^15: an arena of 48 KB
+    wide = [[*range(13)], [*range(2, 13), 13, 14], [0], [14]]
+    diagrams.append(Diagram(Wiring([2] * 15, wide, [*range(14, -1, -1)]),
+                            [(rng.random((2,) * len(ws)) < 0.7).astype(np.uint8) | (len(ws) == 1) for ws in wide]))
     with DeviceRel.mode_scope(mode):
         for i, d in enumerate(diagrams):
             c = PlannedContraction(DeviceRel, d.wiring)
