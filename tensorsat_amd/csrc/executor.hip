@@ -387,7 +387,7 @@ struct GangAny {
 
 // A step in device memory waits for its operands and for its stores to reach L2; in LDS it
 // waits less, so runs long enough to pay for moving their part of the arena there and
-// back are staged (SEQ_STAGE): 16 jobs of 631 steps on the first 15 KB 440 us in place, 400
+// back are staged (seq_staged): 16 jobs of 631 steps on the first 15 KB 440 us in place, 400
 // us staged.
 constexpr int64_t SEQ_LDS = 65536;
 inline bool seq_staged(int steps, int64_t end) { return end <= SEQ_LDS && steps >= 8 && end <= 1024ll * steps; }
