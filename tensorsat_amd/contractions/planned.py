@@ -152,9 +152,14 @@ class SmallTree:
         N = _native
         L = N.lib()
         dev = torch.cuda.current_device()
-        steps = self.device_steps.get(dev)
-        if steps is None:  # a synchronous upload: complete for every stream
-            steps = self.device_steps[dev] = torch.from_numpy(self.prog.steps.view(np.uint8)).cuda()
+        stream = torch.cuda.current_stream()
+        held = self.device_steps.get(dev)
+        if held is None:  # a synchronous upload: complete for every stream
+            held = torch.from_numpy(self.prog.steps.view(np.uint8)).cuda(), stream.cuda_stream
+            self.device_steps[dev] = held
+        steps, owner = held
+        if owner != stream.cuda_stream:  # not given back while this stream still reads it
+            steps.record_stream(stream)
         res = torch.empty(max(16, 1 << self.rank), dtype=torch.uint8, device="cuda")
         N.check(L.ts_program_run_small(N.host_ptr(self.prog.jobs), N.host_ptr(self.prog.steps), N.dptr(steps),
                                        N.host_ptr(bits), N.dptr(res), N.MODES[mode], N.stream_ptr()),
@@ -164,6 +169,11 @@ class SmallTree:
 
 class PlannedContraction(Contraction):
     """A contraction along a planned binary tree (``CotengraContraction`` counterpart)."""
+
+    _small = False  # SmallTree or None, built on the first contraction of host leaves
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != "_small"}  # holds device memory
 
     def __init__(self, box_class: type, wiring: Wiring, *, optimize: str = "auto",
                  slicing_target: float | None = None, trials: int = 32, seed: int = 0,
@@ -175,7 +185,6 @@ class PlannedContraction(Contraction):
         if slicing_target is not None and tree.cost is not None and tree.cost.log2_max_size > slicing_target:
             tree = _plan.slice_plan(wiring, tree, slicing_target, reconfigure_trials=trials, seed=seed)
         self._tree = tree
-        self._small = False  # SmallTree or None, built on the first contraction
 
     @property
     def tree(self) -> _plan.Plan:

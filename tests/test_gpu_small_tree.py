@@ -3,6 +3,8 @@ Trees that run as one device job (host leaves, every tensor in one workgroup's L
 the walk node by node and the oracle, and the diagrams that have to take the walk.
 """
 
+import pickle
+
 import numpy as np
 import pytest
 
@@ -109,3 +111,6 @@ def test_device_blocks_and_other_streams():
         other = c.contract(d)
     s.synchronize()
     np.testing.assert_array_equal(other.tensor, want)
+    copied = pickle.loads(pickle.dumps(c))  # a saved plan holds no device memory
+    assert copied._small is False
+    np.testing.assert_array_equal(copied.contract(d).tensor, want)
