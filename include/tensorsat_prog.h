@@ -45,9 +45,11 @@ typedef struct {
 #define TS_STEP_NORHS 2   /* unary step (rewire/reduce): rhs is the constant 1 */
 #define TS_STEP_PACKET 4  /* packet form (tsc_packetize): pad[0] = first lane of this step */
 #define TS_STEP_PEND 8    /* packet form: last record of its packet */
-/* Counting (tsc_count_widths): pad[0] of a step holds the storage of its operands (bits 0-1
- * lhs, 2-3 rhs: 0 uint64, 1 uint32, 2 uint64 with values below 2^32) and these bits;
- * 0 means uint64 throughout, checked. */
+#define TS_STEP_WIDTHS 16 /* counting (tsc_count_widths): pad[0] = storage widths, TS_COUNT_* */
+/* pad[0] of a TS_STEP_WIDTHS step holds the storage of its operands (bits 0-1 lhs, 2-3 rhs: 0
+ * uint64, 1 uint32, 2 uint64 with values below 2^32) and these bits.  Steps without the flag
+ * are counted in uint64 throughout, checked, whatever pad holds.  A step has this flag or
+ * TS_STEP_PACKET, never both: each gives pad[0] its meaning. */
 #define TS_COUNT_OUT32 16 /* the result is stored as uint32 */
 #define TS_COUNT_EXACT 32 /* no product or sum of this step reaches 2^64 */
 #define TS_PACKET_LANES 64 /* lanes of one packet (one wavefront) */
@@ -157,11 +159,12 @@ int tsc_packetize(ts_job* jobs, int64_t num_jobs, ts_step* steps, int64_t num_st
 
 /* Storage widths of a counting program (no counterpart in the reference: an execution layout
  * of this build): a tensor's entries are at most 2^b, b = the summed bits of all steps under
- * it (plus 8 per leaf if the job has a leaf byte above 1).  Writes pad[0] of every step
- * (TS_COUNT_*); the tensor at a job's result_off stays uint64, and so does every step of a
- * job whose operands are not whole tensors written before (pad[0] = 0).  Offsets and arena
- * sizes stay as they are: a uint32 tensor fills half its room.  threads <= 0: hardware
- * concurrency. */
+ * it (plus 8 per leaf if the job has a leaf byte above 1).  Writes pad[0] (TS_COUNT_*) and
+ * TS_STEP_WIDTHS of every step; the tensor at a job's result_off stays uint64, and so does
+ * every step of a job whose operands are not whole tensors written before (no flag, pad[0] =
+ * 0).  Records in packet form leave it: TS_STEP_PACKET and TS_STEP_PEND are cleared, so only
+ * the counting kernels and the step runners take the program.  Offsets and arena sizes stay
+ * as they are: a uint32 tensor fills half its room.  threads <= 0: hardware concurrency. */
 int tsc_count_widths(const ts_job* jobs, int64_t num_jobs, ts_step* steps, int64_t num_steps,
                      const uint8_t* leaves, int64_t num_leaf_bytes, int32_t threads);
 

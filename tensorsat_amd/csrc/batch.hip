@@ -476,8 +476,8 @@ __global__ __launch_bounds__(64) void k_batch_wave(ts_batch b) {
 // The same walk over (+, x) with exact integer counts: an arena element is 8 bytes wide, and
 // a tensor whose record proves its entries below 2^32 (tsc_count_widths: at most 2^b with b
 // the summed bits under it) is stored as uint32 at the start of its room, so a step reads and
-// writes half the bytes.  Records without that proof (pad[0] = 0) are uint64 with checked
-// arithmetic.  Bound by memory traffic: a width-18 job's arena is 1.3 MB and 1536 of them are
+// writes half the bytes.  Records without that proof (no TS_STEP_WIDTHS) are uint64 with
+// checked arithmetic.  Bound by memory traffic: a width-18 job's arena is 1.3 MB and 1536 of them are
 // in flight, far beyond the caches.  n=100, m=300 over 46816 cubes of width 18 (23 G elements
 // read and written): 84 ms with uint64 tensors and one thread per output, 66 ms with uint32
 // ones (the longest sums of 2^16 terms on one thread then hold their job for 40 ms), 51 ms
@@ -715,7 +715,7 @@ __global__ __launch_bounds__(CWG) void k_batch_count(ts_batch b, unsigned long l
       __syncthreads();
       for (int s = 0; s < ns; ++s) {
         const ts_step& st = s_steps[s];
-        const CountTag tag{st.pad[0]};
+        const CountTag tag{(st.flags & TS_STEP_WIDTHS) ? st.pad[0] : 0u};  // packet form: pad[0] is a lane
         const bool kinner = st.flags & TS_STEP_KINNER, norhs = st.flags & TS_STEP_NORHS;
         uint8_t* base = reinterpret_cast<uint8_t*>(arena);
         const uint8_t* lhs = base + 8ull * st.lhs_off;

@@ -144,7 +144,7 @@ int packetize_job(ts_job& job, ts_step* st) {
       if (pl[i] >= 0) r.lhs_off = (uint32_t)noff[pl[i]];
       if (pr[i] >= 0) r.rhs_off = (uint32_t)noff[pr[i]];
       if (r.flags & TS_STEP_NORHS) r.rhs_off = r.lhs_off;
-      r.flags |= TS_STEP_PACKET;
+      r.flags = (uint8_t)((r.flags & ~TS_STEP_WIDTHS) | TS_STEP_PACKET);
       r.pad[0] = (uint8_t)lane;
       mask |= uint64_t(1) << lane;
       lane += lanes[i];
@@ -257,8 +257,12 @@ extern "C" int tsc_count_widths(const ts_job* jobs, int64_t num_jobs, ts_step* s
         jobs[j].leaf_begin < 0 || jobs[j].num_leaf_bytes < 0 ||
         jobs[j].leaf_begin + jobs[j].num_leaf_bytes > num_leaf_bytes)
       return TSP_EINVAL;
+  for (int64_t i = 0; i < num_steps; ++i) {  // leave the packet form: lanes and lane masks
+    if (steps[i].flags & TS_STEP_PACKET) std::memset(&steps[i].o_lpos[16], TS_NOPOS, 8);
+    steps[i].pad[0] = 0;
+    steps[i].flags &= (uint8_t)~(TS_STEP_WIDTHS | TS_STEP_PACKET | TS_STEP_PEND);
+  }
   // Jobs that share step records must agree on their tags: such programs stay uint64.
-  for (int64_t i = 0; i < num_steps; ++i) steps[i].pad[0] = 0;
   std::vector<uint8_t> used((size_t)num_steps, 0);
   for (int64_t j = 0; j < num_jobs; ++j)
     for (int32_t i = 0; i < jobs[j].num_steps; ++i)
@@ -271,7 +275,10 @@ extern "C" int tsc_count_widths(const ts_job* jobs, int64_t num_jobs, ts_step* s
     for (int64_t j = t; j < num_jobs; j += nt) {
       ts_step* st = steps + jobs[j].step_begin;
       if (!count_widths_job(jobs[j], st, leaves, table, tags)) continue;
-      for (int32_t i = 0; i < jobs[j].num_steps; ++i) st[i].pad[0] = tags[i];
+      for (int32_t i = 0; i < jobs[j].num_steps; ++i) {
+        st[i].pad[0] = tags[i];
+        st[i].flags |= TS_STEP_WIDTHS;
+      }
     }
   };
   std::vector<std::thread> pool;

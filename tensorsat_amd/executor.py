@@ -429,7 +429,8 @@ class BatchExecutor:
 class BatchCounter:
     """
     Exact model counts of all jobs of a program in one persistent launch
-    (``ts_batch_count``): uint64 arenas, per-instance sums of result x 2^free_vars,
+    (``ts_batch_count``): tensors stored as uint32 where their entries provably fit and as
+    uint64 elsewhere (:func:`program.count_widths`), per-instance sums of result x 2^free_vars,
     overflow flags raised instead of wrapping.
     """
 

@@ -25,6 +25,7 @@ STEP_KINNER = 1
 STEP_NORHS = 2
 STEP_PACKET = 4  # packet form (packetize): pad[0] = first lane of the step
 STEP_PEND = 8  # packet form: last record of its packet
+STEP_WIDTHS = 16  # counting (count_widths): pad[0] = storage widths
 PACKET_LANES = 64
 PACKET_CHUNK = 16
 NSTAT = 10
@@ -414,13 +415,15 @@ def count_widths(prog: Program, threads: int = 0) -> Program:
     """
     ``prog`` with the storage width of every counting step in its record
     (``tsc_count_widths``): tensors whose entries are provably below 2^32 are held as
-    uint32 by the batched counter.  Values are unchanged; returns a new Program.
+    uint32 by the batched counter.  Values are unchanged; returns a new Program, which is no
+    longer in packet form if ``prog`` was (a record holds lanes or widths).
     """
     steps = prog.steps.copy()
     leaves = np.ascontiguousarray(prog.leaves, dtype=np.uint8)
     _plan._check(_lib().tsc_count_widths(prog.jobs.ctypes.data, len(prog.jobs), steps.ctypes.data, len(steps),
                                          leaves.ctypes.data, leaves.size, int(threads)), "tsc_count_widths")
-    return Program(prog.jobs, steps, prog.leaves, prog.stats, dict(prog.meta))
+    meta = {k: v for k, v in prog.meta.items() if k != "packetized"}
+    return Program(prog.jobs, steps, prog.leaves, prog.stats, meta)
 
 
 LANE_DTYPE = np.dtype(

@@ -103,3 +103,40 @@ def test_wide_sums_and_general_steps():
             for side, name in enumerate(("c_lpos", "c_rpos")):
                 at[side] |= ((idx >> k) & 1) << int(prog.steps[name][0, k])
         assert got == [int((lhs[at[0]] * rhs[at[1]]).sum())]
+
+
+def _packet_programs():
+    for width, sizes in ((6, (12, 20, 30)), (4, (16, 22, 24))):
+        yield PG.sat_batch([CNFInstance.random(3, n, 3 * n, rng=n) for n in sizes], width=width)
+
+
+def test_widths_and_lanes_exclude_each_other():
+    for prog in _packet_programs():
+        pk = PG.packetize(prog)
+        assert (pk.steps["pad"][:, 0] > 0).any()  # lanes
+        wide = PG.count_widths(pk)
+        assert not (wide.steps["flags"] & (PG.STEP_PACKET | PG.STEP_PEND)).any()
+        assert (wide.steps["flags"] & PG.STEP_WIDTHS).all() and "packetized" not in wide.meta
+        with pytest.raises(ValueError):
+            PG.lanes(wide)
+        assert (pk.steps["flags"] & PG.STEP_PACKET).all()  # the given program is left alone
+        again = PG.packetize(PG.count_widths(prog))
+        assert not (again.steps["flags"] & PG.STEP_WIDTHS).any()
+        assert (again.steps == pk.steps).all()
+        PG.lanes(again)
+
+
+@pytest.mark.gpu
+def test_records_without_widths_count_as_uint64():
+    """Packet-form records (pad[0] = a lane) and records whose pad was never cleared, through
+    the C entry."""
+    from tensorsat_amd.executor import BatchCounter, DeviceProgram
+
+    for prog in _packet_programs():
+        want = BatchCounter(prog).run()
+        dirty = PG.Program(prog.jobs, prog.steps.copy(), prog.leaves, prog.stats, {})
+        dirty.steps["pad"] = np.random.default_rng(0).integers(0, 256, dirty.steps["pad"].shape)
+        for other in (PG.packetize(prog), dirty):
+            counter = BatchCounter(other)
+            counter.dp = DeviceProgram(other)  # the records as they are
+            assert counter.run() == want
