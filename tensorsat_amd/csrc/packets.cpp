@@ -191,40 +191,66 @@ extern "C" int tsc_packetize(ts_job* jobs, int64_t num_jobs, ts_step* steps, int
 
 namespace {
 
-struct Held {  // the tensor at an arena offset
-  uint32_t off;
-  int rank, bound, kind, step;  // step: the one that wrote it (-1: a leaf)
+struct Held {  // arena entries [off, off + len) as the last write to them left them
+  uint32_t off, len;
+  int step, bound;    // step: the one that wrote them
+  int8_t rank, kind;  // rank -1: what is left of a tensor, a part of it overwritten
+  uint64_t end() const { return (uint64_t)off + len; }
 };
 
-// One job's tags; false if an operand is not a whole tensor written before.
-bool count_widths_job(const ts_job& job, ts_step* st, const uint8_t* leaves, std::vector<Held>& table,
+// Written entries of one job's arena, sorted and disjoint.
+struct HeldSet {
+  std::vector<Held> v;
+
+  size_t first_past(uint64_t off) const {  // first entry that ends after off
+    return std::upper_bound(v.begin(), v.end(), off, [](uint64_t o, const Held& h) { return o < h.end(); }) - v.begin();
+  }
+  // The tensor that fills [off, off + 2^rank); *touched: anything was written there.
+  const Held* find(uint64_t off, int rank, bool* touched) const {
+    const size_t i = first_past(off);
+    *touched = i < v.size() && v[i].off < off + (1ull << rank);
+    return *touched && v[i].off == off && v[i].rank == rank ? &v[i] : nullptr;
+  }
+  void write(const Held& h) {
+    const size_t i = first_past(h.off);
+    size_t j = i;
+    while (j < v.size() && v[j].off < h.end()) ++j;
+    Held keep[3];
+    size_t n = 0;
+    if (i < j && v[i].off < h.off) keep[n++] = Held{v[i].off, h.off - v[i].off, 0, 0, -1, 0};
+    keep[n++] = h;
+    if (i < j && v[j - 1].end() > h.end())
+      keep[n++] = Held{(uint32_t)h.end(), (uint32_t)(v[j - 1].end() - h.end()), 0, 0, -1, 0};
+    const size_t m = std::min(n, j - i);  // overwritten in place
+    std::copy(keep, keep + m, v.begin() + (long)i);
+    if (n > m) v.insert(v.begin() + (long)(i + m), keep + m, keep + n);
+    else v.erase(v.begin() + (long)(i + m), v.begin() + (long)j);
+  }
+};
+
+// One job's tags; false if an operand or the result is not a whole tensor written before (or
+// leaf entries that no step wrote to).
+bool count_widths_job(const ts_job& job, ts_step* st, const uint8_t* leaves, HeldSet& held,
                       std::vector<uint8_t>& tags) {
   const int n = job.num_steps;
-  size_t cap = 64;
-  while (cap < 4u * (size_t)(n + 1)) cap *= 2;
-  table.assign(cap, Held{UINT32_MAX, 0, 0, 0, 0});
-  auto slot = [&](uint32_t off) -> Held& {
-    size_t h = (off * 0x9e3779b1u) & (cap - 1);
-    while (table[h].off != UINT32_MAX && table[h].off != off) h = (h + 1) & (cap - 1);
-    return table[h];
-  };
+  held.v.clear();
   int leaf_bits = 0;
   for (int32_t i = 0; i < job.num_leaf_bytes; ++i)
     if (leaves[job.leaf_begin + i] > 1) leaf_bits = 8;
   tags.assign(n, 0);
+  bool touched;
   for (int i = 0; i < n; ++i) {
     const ts_step& s = st[i];
     int bound = s.sum_rank, kinds[2] = {0, 0};
     for (int side = 0; side < ((s.flags & TS_STEP_NORHS) ? 1 : 2); ++side) {
       const uint32_t off = side ? s.rhs_off : s.lhs_off;
       const int rank = side ? s.rhs_rank : s.lhs_rank;
-      const Held& h = slot(off);
-      if (h.off == off) {
-        if (h.rank != rank) return false;
-        bound += h.bound;
-        kinds[side] = h.kind;
+      const Held* h = held.find(off, rank, &touched);
+      if (h) {
+        bound += h->bound;
+        kinds[side] = h->kind;
       } else {
-        if ((uint64_t)off + (1ull << rank) > (uint64_t)job.num_leaf_bytes) return false;
+        if (touched || (uint64_t)off + (1ull << rank) > (uint64_t)job.num_leaf_bytes) return false;
         bound += leaf_bits;
         kinds[side] = 2;  // leaves are copied as uint64
       }
@@ -232,15 +258,15 @@ bool count_widths_job(const ts_job& job, ts_step* st, const uint8_t* leaves, std
     // values up to 2^bound: uint32 holds 2^31, uint64 holds 2^63
     const bool narrow = bound <= 31, exact = bound <= 63;
     tags[i] = (uint8_t)(kinds[0] | (kinds[1] << 2) | (narrow ? TS_COUNT_OUT32 : 0) | (exact ? TS_COUNT_EXACT : 0));
-    slot(s.out_off) = Held{s.out_off, s.out_rank, bound, narrow ? 1 : 0, i};
+    held.write(Held{s.out_off, 1u << s.out_rank, i, bound, (int8_t)s.out_rank, (int8_t)(narrow ? 1 : 0)});
   }
-  // The result is read as uint64; it is the last tensor at its offset, so no step reads it.
-  const Held& res = slot((uint32_t)job.result_off);
-  if (res.off == (uint32_t)job.result_off) {
-    if (res.rank != job.result_rank) return false;
-    for (int i = res.step + 1; i < n; ++i)
-      if (st[i].lhs_off == res.off || (!(st[i].flags & TS_STEP_NORHS) && st[i].rhs_off == res.off)) return false;
-    tags[res.step] &= (uint8_t)~TS_COUNT_OUT32;
+  // The result is read as uint64; it is the last tensor at its place, so no step reads it.
+  const Held* res = held.find((uint64_t)job.result_off, job.result_rank, &touched);
+  if (touched && !res) return false;
+  if (res) {
+    for (int i = res->step + 1; i < n; ++i)
+      if (st[i].lhs_off == res->off || (!(st[i].flags & TS_STEP_NORHS) && st[i].rhs_off == res->off)) return false;
+    tags[res->step] &= (uint8_t)~TS_COUNT_OUT32;
   }
   return true;
 }
@@ -270,11 +296,11 @@ extern "C" int tsc_count_widths(const ts_job* jobs, int64_t num_jobs, ts_step* s
   int nt = threads > 0 ? threads : (int)std::max(1u, std::thread::hardware_concurrency());
   nt = (int)std::max<int64_t>(1, std::min<int64_t>(nt, num_jobs / 64 + 1));
   auto work = [&](int t) {
-    std::vector<Held> table;
+    HeldSet held;
     std::vector<uint8_t> tags;
     for (int64_t j = t; j < num_jobs; j += nt) {
       ts_step* st = steps + jobs[j].step_begin;
-      if (!count_widths_job(jobs[j], st, leaves, table, tags)) continue;
+      if (!count_widths_job(jobs[j], st, leaves, held, tags)) continue;
       for (int32_t i = 0; i < jobs[j].num_steps; ++i) {
         st[i].pad[0] = tags[i];
         st[i].flags |= TS_STEP_WIDTHS;

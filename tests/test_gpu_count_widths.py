@@ -105,6 +105,57 @@ def test_wide_sums_and_general_steps():
         assert got == [int((lhs[at[0]] * rhs[at[1]]).sum())]
 
 
+def _steps_by_hand(kind):
+    """128 leaf entries of ones, tensors written over them, one operand (or the result) that is a
+    part of a tensor; and the count."""
+    copy = lambda lhs, rank, out: (lhs, out, rank, rank)
+    total = lambda lhs, rank, out: (lhs, out, rank, 0)
+    rows = {
+        # the upper half of a tensor of 32 at 32
+        "upper half": [copy(0, 5, 32), total(48, 4, 128)],
+        # a tensor at 48, then a larger one over it, whose upper half is read there
+        "overwritten": [copy(0, 4, 48), copy(0, 5, 32), total(48, 4, 128)],
+        # the lower half of a tensor whose upper half was overwritten
+        "remains": [copy(0, 5, 32), copy(0, 4, 48), total(32, 4, 128)],
+        # the result is the middle entry of a tensor
+        "result": [copy(0, 5, 112)],
+        "whole": [copy(0, 4, 32), copy(0, 4, 48), total(48, 4, 128)],
+    }[kind]
+    steps = np.zeros(len(rows), PG.STEP_DTYPE)
+    for name in ("o_lpos", "o_rpos", "c_lpos", "c_rpos"):
+        steps[name] = PG.NOPOS
+    for st, (lhs, out, rank, ro) in zip(steps, rows):
+        st["lhs_off"], st["rhs_off"], st["out_off"] = lhs, lhs, out
+        st["lhs_rank"], st["out_rank"], st["sum_rank"] = rank, ro, rank - ro
+        st["flags"] = PG.STEP_NORHS | PG.STEP_KINNER
+        st["o_lpos"][:ro] = range(ro)
+        st["c_lpos"][: rank - ro] = range(rank - ro)
+    jobs = np.zeros(1, PG.JOB_DTYPE)
+    jobs["num_steps"], jobs["num_leaf_bytes"], jobs["result_off"], jobs["arena_elems"] = len(rows), 128, 128, 160
+    want = 1 if kind == "result" else 16
+    return PG.Program(jobs, steps, np.ones(128, np.uint8), np.zeros((1, PG.NSTAT), np.int64), {}), want
+
+
+@pytest.mark.parametrize("kind", ["upper half", "overwritten", "remains", "result", "whole"])
+def test_parts_of_tensors_stay_uint64(kind):
+    prog, _ = _steps_by_hand(kind)
+    PG.validate(prog)
+    got = PG.count_widths(prog).steps
+    if kind == "whole":
+        assert [int(t) for t in got["pad"][:, 0]] == [2 | OUT32 | EXACT, 2 | OUT32 | EXACT, 1 | EXACT]
+    else:
+        assert not got["pad"].any() and not (got["flags"] & PG.STEP_WIDTHS).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["upper half", "overwritten", "remains", "result", "whole"])
+def test_counts_over_parts_of_tensors(kind):
+    from tensorsat_amd.executor import BatchCounter
+
+    prog, want = _steps_by_hand(kind)
+    assert BatchCounter(prog).run() == [want]
+
+
 def _packet_programs():
     for width, sizes in ((6, (12, 20, 30)), (4, (16, 22, 24))):
         yield PG.sat_batch([CNFInstance.random(3, n, 3 * n, rng=n) for n in sizes], width=width)
