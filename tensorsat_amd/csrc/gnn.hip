@@ -802,7 +802,7 @@ int launch_panel(const void* A, int64_t lda, const void* B, int64_t sbk, int64_t
 
 // Blocks of rows of a weight gradient: one per 256 rows, up to a workgroup per CU.
 inline int wgrad_blocks(int M, int rows) {
-  const int mtiles = (M + WM - 1) / WM;
+  const int mtiles = std::max(1, (M + WM - 1) / WM);
   return std::max(1, std::min((rows + 255) / 256, 256 / mtiles));
 }
 

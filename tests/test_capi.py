@@ -65,3 +65,18 @@ def test_dense_tile_table_host_side():
     assert L.ts_dense_tiles(8, 8, 0, 8, 7) == N.TS_EINVAL
     assert L.ts_dense_tiles(-1, 8, 0, 8, 1) == N.TS_EINVAL
     assert L.ts_dense_tile_of(8, 8, 0, 28, None) == N.TS_EINVAL
+
+
+def test_weight_gradient_scratch_sizes():
+    """Host arithmetic only: no columns or rows need no scratch, a multiple of 64 KiB per tile
+    otherwise, sizes out of range refused."""
+    from tensorsat_amd import _native as N
+
+    L = N.load()
+    need = N.i64(-1)
+    for m, rows, blocks in ((0, 0, 0), (0, 1000, 0), (1, 0, 1), (128, 1, 1), (132, 257, 4), (32768, 10**6, 256)):
+        assert L.ts_gnn_wgrad_scratch(m, rows, ctypes.byref(need)) == 0
+        assert need.value == blocks * 128 * 128 * 4, (m, rows)
+    for m, rows in ((-1, 5), (5, -1), (32769, 5)):
+        assert L.ts_gnn_wgrad_scratch(m, rows, ctypes.byref(need)) == N.TS_EINVAL
+    assert L.ts_gnn_wgrad_scratch(4, 4, None) == N.TS_EINVAL
