@@ -103,10 +103,11 @@ class SmallTree:
     # per step: a step of 2^14 products takes them about 4 us, the walk 35 us of host.
     MAX_TERMS = 1 << 14
 
-    @classmethod
-    def build(cls, wiring: Wiring, tree: _plan.Plan) -> "SmallTree | None":
-        """None where the walk has to run: sliced trees, extents other than 2, repeated or
-        dangling wires, a single slot, or tensors that do not fit one workgroup."""
+    @staticmethod
+    def slot_shapes(wiring: Wiring, tree: _plan.Plan) -> list[tuple[int, ...]] | None:
+        """The leaves' shapes; None where the wiring or the tree has to take the walk: sliced
+        trees, extents other than 2, repeated or dangling wires, a single slot, or leaves that
+        do not fit one workgroup."""
         slots, outs = wiring.slot_wires_list, wiring.out_wires
         if len(slots) < 2 or len(tree.sliced) or any(d != 2 for d in wiring.wire_dims):
             return None
@@ -115,35 +116,52 @@ class SmallTree:
             return None
         if sum(1 << len(ws) for ws in slots) > _native.SMALL_LEAVES:
             return None
-        cost = _plan.tree_cost(wiring, tree)
-        if cost.log2_max_size > 15:
+        return [(2,) * len(ws) for ws in slots]
+
+    @classmethod
+    def build(cls, wiring: Wiring, tree: _plan.Plan, shapes=None) -> "SmallTree | None":
+        """None where the walk has to run (:meth:`slot_shapes`, or tensors that do not fit one
+        workgroup)."""
+        shapes = shapes or cls.slot_shapes(wiring, tree)
+        if shapes is None or _plan.tree_cost(wiring, tree).log2_max_size > 15:
             return None
         # The compiler lays leaf entries out in its own order: compiled with each entry's
         # index (its low, then its high byte) as the value, the leaves say which goes where.
-        sizes = [1 << len(ws) for ws in slots]
+        sizes = [1 << len(shape) for shape in shapes]
         index = np.split(np.arange(sum(sizes)), np.cumsum(sizes)[:-1])
-        lo, hi = (_prog.compile_network(wiring, [((ix >> sh) & 255).astype(np.uint8) for ix in index], tree)
-                  for sh in (0, 8))
+
+        def compiled(shift: int) -> _prog.Program:
+            return _prog.compile_network(wiring, [((ix >> shift) & 255).astype(np.uint8) for ix in index], tree)
+
+        lo = compiled(0)
         terms = np.ldexp(1.0, lo.steps["out_rank"].astype(int) + lo.steps["sum_rank"]).sum()
         if (len(lo.jobs) != 1 or int(lo.jobs["arena_elems"][0]) > _native.SMALL_ARENA or
                 lo.leaves.size > _native.SMALL_LEAVES or terms > cls.MAX_TERMS * len(lo.steps)):
             return None
+        high = compiled(8).leaves.astype(np.int64) << 8 if sum(sizes) > 256 else 0
         self = object.__new__(cls)
         self.prog = lo
-        self.source = lo.leaves.astype(np.int64) | (hi.leaves.astype(np.int64) << 8)
-        self.shapes = [(2,) * len(ws) for ws in slots]
-        self.rank = len(outs)
+        self.source = lo.leaves.astype(np.int64) | high
+        self.shapes = shapes
+        self.rank = len(wiring.out_wires)
         self.device_steps = {}
         return self
 
-    def leaf_bits(self, blocks) -> np.ndarray | None:
-        """The job's leaves as bits, or None if the blocks are not 0/1 host arrays of the
+    @staticmethod
+    def entries(shapes, blocks) -> np.ndarray | None:
+        """All leaf entries in slot order, or None if the blocks are not 0/1 host arrays of the
         slots' shapes."""
-        if not all(type(b) is np.ndarray for b in blocks) or [b.shape for b in blocks] != self.shapes:
+        if not all(type(b) is np.ndarray for b in blocks) or [b.shape for b in blocks] != shapes:
             return None
         flat = np.concatenate([b.reshape(-1) for b in blocks])
-        if flat.dtype != np.uint8 or flat.max() > 1:
-            return None
+        return flat if flat.dtype == np.uint8 and flat.max() <= 1 else None
+
+    def leaf_bits(self, blocks) -> np.ndarray | None:
+        """The job's leaves as bits, or None where :meth:`entries` is."""
+        flat = self.entries(self.shapes, blocks)
+        return None if flat is None else self.pack(flat)
+
+    def pack(self, flat: np.ndarray) -> np.ndarray:
         return np.packbits(flat[self.source], bitorder="little")
 
     def run(self, bits: np.ndarray, box_class, mode: str):
@@ -170,7 +188,7 @@ class SmallTree:
 class PlannedContraction(Contraction):
     """A contraction along a planned binary tree (``CotengraContraction`` counterpart)."""
 
-    _small = False  # SmallTree or None, built on the first contraction of host leaves
+    _small = False  # SmallTree or None, built on the first contraction of 0/1 host leaves
 
     def __getstate__(self):
         return {k: v for k, v in self.__dict__.items() if k != "_small"}  # holds device memory
@@ -236,13 +254,25 @@ class PlannedContraction(Contraction):
             wires = wires + dangling
         return box, wires
 
+    def _small_bits(self, blocks) -> np.ndarray | None:
+        """The leaves as bits of the tree's small job, or None where the walk runs.  The job is
+        laid out (two compilations, a few ms) only for leaves that it takes."""
+        small = self._small
+        if small is None:
+            return None
+        shapes = small.shapes if small else SmallTree.slot_shapes(self.wiring, self._tree)
+        flat = SmallTree.entries(shapes, blocks) if shapes else None
+        if flat is None:
+            return None
+        if small is False:
+            small = self._small = SmallTree.build(self.wiring, self._tree, shapes)
+        return None if small is None else small.pack(flat)
+
     def contract(self, diagram: Diagram, *, order=None, autojit="auto", progbar: bool = False):
         """Validate and contract (``cotengra.py:100-128``)."""
         self.validate(diagram)
         if self.box_class is DeviceRel:
-            if self._small is False:
-                self._small = SmallTree.build(self.wiring, self._tree)
-            bits = self._small.leaf_bits(diagram.blocks) if self._small is not None else None
+            bits = self._small_bits(diagram.blocks)
             if bits is not None:
                 return self._small.run(bits, DeviceRel, DeviceRel._mode)
         boxes = self._boxes(diagram)

@@ -62,6 +62,67 @@ def test_trees_that_take_the_walk():
                 assert (got[off : off + (1 << rank)] == prog.leaves[off : off + (1 << rank)]).all()
 
 
+def test_jobs_are_laid_out_for_host_leaves_only(monkeypatch):
+    """Leaves that take the walk never reach the compiler."""
+    from tensorsat_amd.rel import DeviceRel
+
+    leaf, wide = np.ones((2, 2), np.uint8), np.ones((2,) * 15, np.uint8)
+    for wires, blocks in (
+        ([[0, 1], [1, 2]], [leaf, object()]), ([[0, 1], [1, 2]], [object(), object()]),
+        ([[0, 1], [1, 2]], [leaf, 2 * leaf]), ([[0, 1], [1, 2]], [leaf.astype(bool)] * 2),
+        ([[0, 1], [1, 2]], [leaf, leaf[0]]), ([[*range(15)], [*range(1, 16)]], [wide, wide]),
+    ):
+        w = Wiring([2] * (1 + max(max(ws) for ws in wires)), wires, [0])
+        c = PlannedContraction(DeviceRel, w)
+        monkeypatch.setattr(SmallTree, "build", lambda *a: pytest.fail("laid out"))
+        assert c._small_bits(blocks) is None and c._small is False
+        monkeypatch.undo()
+        host = [np.ones((2,) * len(ws), np.uint8) for ws in wires]
+        bits = c._small_bits(host)  # 2^16 leaf entries are too many
+        assert (bits is None) == (len(wires[0]) == 15) and (c._small is False) == (bits is None)
+
+
+def _walk(wiring, tree, blocks, mode):
+    """The tree's steps one by one in numpy, the result in out-wire order."""
+    from tensorsat_amd.contractions.planned import tree_steps
+
+    live = {i: (b.astype(np.int64), list(ws)) for i, (b, ws) in enumerate(zip(blocks, wiring.slot_wires_list))}
+    for k, (a, b, _, _, out) in enumerate(tree_steps(wiring, tree.path)[0]):
+        (x, lx), (y, ly) = live.pop(a), live.pop(b)
+        ids = {w: i for i, w in enumerate(dict.fromkeys(lx + ly))}
+        cnt = np.einsum(x, [ids[w] for w in lx], y, [ids[w] for w in ly], [ids[w] for w in out])
+        live[wiring.num_slots + k] = (cnt % 256 if mode == "MOD256" else cnt).astype(bool).astype(np.int64), list(out)
+    ((r, ws),) = live.values()
+    return r.transpose([ws.index(w) for w in wiring.out_wires]).reshape(-1)
+
+
+@pytest.mark.parametrize("mode", ["GT0", "MOD256"])
+def test_job_equals_the_walk_on_any_wiring(mode):
+    """The job's records and leaves, run by the oracle: scalar slots, unheld wires, wires summed
+    in one slot, unconnected parts, any out order."""
+    from oracle import executor as OX
+    from tensorsat_amd import program as PG
+
+    rng, taken = np.random.default_rng(3), 0
+    for i in range(200):
+        n = int(rng.integers(1, 14))
+        ws = [[int(w) for w in rng.choice(n, size=min(n, int(rng.integers(0, 6))), replace=False)]
+              for _ in range(int(rng.integers(2, 14)))]
+        held = sorted({w for s in ws for w in s})
+        w = Wiring([2] * n, ws, [int(x) for x in rng.permutation(held)[: int(rng.integers(0, 7))]])
+        blocks = [np.asarray(rng.random((2,) * len(s)) < (0.95 if i % 3 else 1.1)).astype(np.uint8).reshape((2,) * len(s))
+                  for s in ws]
+        c = PlannedContraction(OracleRel, w)
+        t = SmallTree.build(w, c.tree)
+        if t is None:
+            continue
+        taken += 1
+        leaves = np.unpackbits(t.leaf_bits(blocks), bitorder="little")[: t.prog.leaves.size]
+        got, _ = OX.run_job(PG.Program(t.prog.jobs, t.prog.steps, leaves, t.prog.stats, {}), 0, mode)
+        np.testing.assert_array_equal(np.asarray(got).reshape(-1), _walk(w, c.tree, blocks, mode), err_msg=f"{ws}")
+    assert taken > 150
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["GT0", "MOD256"])
 def test_small_trees_match_the_walk_and_the_oracle(mode):
