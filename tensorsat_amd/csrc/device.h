@@ -164,28 +164,30 @@ __device__ __forceinline__ uint64_t load_row(const uint8_t* p, int nc) {
 
 // ---- vector path for short rows ------------------------------------------------------
 //
-// Rows of 1..8 bytes (at most 3 summed bits, innermost).  Where each operand holds the two
-// lowest out bits right above its summed bits in order (or not at all) -- the compiler lays
-// out every operand so -- the rows of 4 consecutive outputs are one run of at most 32 bytes.
-// A lane computes 16 consecutive outputs as four such groups: out bits 2 and 3 just move the
-// run's address, so all its loads go out at once, and the rows are combined a dword at a
-// time (v_perm picks the four outputs' bytes of one term; rows of 4 and 8 bytes are whole
-// dwords).  Counts are at most 64, so both epilogues reduce to "any bit of the AND set".
+// Rows of 1..8 bytes (at most 3 summed bits, innermost).  Where each operand holds the T
+// lowest out bits right above its summed bits in order (or not at all), the rows of 2^T
+// consecutive outputs are one run of at most 32 bytes; T = 2 for every layout of the compiler,
+// T = 1 only for operands that come in other orders.  A lane computes 16 consecutive outputs
+// as groups of 2^T: the other low out bits just move the run's address, so all its loads go
+// out at once, and the rows are combined a dword at a time (v_perm picks the bytes of one term
+// of four outputs; rows of 4 and 8 bytes are whole dwords).  Counts are at most 64, so both
+// epilogues reduce to "any bit of the AND set".
 // Bound by HBM and, on many workgroups, by their tables: 16 jobs of 2^23 outputs on 65536
 // workgroups took 336 us with each output's row picked out of a chunk held in 64-bit words
 // (40 vector instructions per output), 288 us with dwords (6), and 75 us once 8192 workgroups
 // shared the work.
 
-__host__ __device__ inline bool quad_shaped(const ts_step& st) {
+// T of a step (2 or 1), 0 if it has no such runs.
+__host__ __device__ inline int run_bits(const ts_step& st) {
   const int nc = st.sum_rank;
-  if (nc > 3 || !(nc == 0 || (st.flags & TS_STEP_KINNER)) || st.out_rank < 4) return false;
+  if (nc > 3 || !(nc == 0 || (st.flags & TS_STEP_KINNER)) || st.out_rank < 4) return 0;
   const bool norhs = st.flags & TS_STEP_NORHS;
   int hl = 0, hr = 0;
   for (int j = 0; j < 2; ++j) {
-    if (st.o_lpos[j] != TS_NOPOS && st.o_lpos[j] != nc + hl++) return false;
-    if (!norhs && st.o_rpos[j] != TS_NOPOS && st.o_rpos[j] != nc + hr++) return false;
+    if (st.o_lpos[j] != TS_NOPOS && st.o_lpos[j] != nc + hl++) return j;
+    if (!norhs && st.o_rpos[j] != TS_NOPOS && st.o_rpos[j] != nc + hr++) return j;
   }
-  return true;
+  return 2;
 }
 
 // 2^LG bytes (LG <= 5) as dwords.
@@ -218,47 +220,52 @@ __device__ __forceinline__ Run<LG> load_run(const uint8_t* p) {
   return r;
 }
 
-// Index of output i's row in an operand that holds H of the two lowest out bits (H = 1: bit
+// Index of output i's row in an operand that holds H of the T lowest out bits (H = 1 of 2: bit
 // `one` of them).
-template <int H>
-__device__ __forceinline__ uint32_t quad_row(int i, int one) {
-  return H == 0 ? 0u : H == 2 ? (uint32_t)i : (uint32_t)(i >> one) & 1u;
+template <int T, int H>
+__device__ __forceinline__ uint32_t run_row(int i, int one) {
+  return H == 0 ? 0u : H == T ? (uint32_t)i : (uint32_t)(i >> one) & 1u;
 }
 
-// Byte c of the four outputs' rows (K <= 1).
-template <int K, int H>
-__device__ __forceinline__ uint32_t quad_bytes(const Run<K + H>& r, uint32_t sel, int c) {
-  return __builtin_amdgcn_perm(r.w[1], r.w[0], sel + 0x01010101u * (uint32_t)c);
+// Byte c of the rows of outputs 4d .. 4d + 3 (K <= 1): of one run (T = 2), or of two runs of at
+// most a dword each, side by side (T = 1).
+template <int T, class R>
+__device__ __forceinline__ uint32_t run_bytes(const R* r, int d, uint32_t sel, int c) {
+  const uint32_t lo = T == 2 ? r[d].w[0] : r[2 * d].w[0], hi = T == 2 ? r[d].w[1] : r[2 * d + 1].w[0];
+  return __builtin_amdgcn_perm(hi, lo, sel + 0x01010101u * (uint32_t)c);
 }
 
-// Dword d of output i's row (K >= 2).
-template <int K, int H>
-__device__ __forceinline__ uint32_t quad_word(const Run<K + H>& r, int i, int d, int one) {
+// Dword d of output i's row within its run (K >= 2).
+template <int T, int K, int H>
+__device__ __forceinline__ uint32_t run_word(const Run<K + H>& r, int i, int d, int one) {
   constexpr int D = 1 << (K - 2);
-  if constexpr (H == 1) return one ? r.w[(i >> 1) * D + d] : r.w[(i & 1) * D + d];
+  if constexpr (H == 1 && T == 2) return one ? r.w[(i >> 1) * D + d] : r.w[(i & 1) * D + d];
   else return r.w[(H == 0 ? 0 : i) * D + d];
 }
 
-template <int K, int HL, int HR, int NQ>
-__device__ void step_quad_kh(const ts_step& st, const LutT<NQ>& L, const uint8_t* __restrict__ lhs,
+template <int T, int K, int HL, int HR, int NQ>
+__device__ void step_runs_kh(const ts_step& st, const LutT<NQ>& L, const uint8_t* __restrict__ lhs,
                              const uint8_t* __restrict__ rhs, uint8_t* __restrict__ out, uint64_t first,
                              uint64_t stride) {
+  constexpr int G = 16 >> T, B = 4 - T;  // runs per operand, out bits that tell them apart
   const bool norhs = st.flags & TS_STEP_NORHS;
   const int nqo = nchunks(st.out_rank);
   const uint64_t n = 1ull << (st.out_rank - 4);
   if (first >= n) return;
   const int one_l = st.o_lpos[0] == TS_NOPOS, one_r = norhs || st.o_rpos[0] == TS_NOPOS;
-  uint32_t dl[2], dr[2];  // what out bits 2 and 3 add to the offsets
+  uint32_t dl[B], dr[B];  // what out bits T .. 3 add to the offsets
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    dl[j] = st.o_lpos[2 + j] != TS_NOPOS ? 1u << st.o_lpos[2 + j] : 0u;
-    dr[j] = !norhs && st.o_rpos[2 + j] != TS_NOPOS ? 1u << st.o_rpos[2 + j] : 0u;
+  for (int j = 0; j < B; ++j) {
+    dl[j] = st.o_lpos[T + j] != TS_NOPOS ? 1u << st.o_lpos[T + j] : 0u;
+    dr[j] = !norhs && st.o_rpos[T + j] != TS_NOPOS ? 1u << st.o_rpos[T + j] : 0u;
   }
   uint32_t sl = 0, sr = 0;  // byte selectors of term 0 (K <= 1)
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    sl |= (quad_row<HL>(i, one_l) << K) << (8 * i);
-    sr |= (quad_row<HR>(i, one_r) << K) << (8 * i);
+    const uint32_t run = T == 2 ? 0u : 4u * (uint32_t)(i >> 1);
+    const int k = i & ((1 << T) - 1);
+    sl |= (run + (run_row<T, HL>(k, one_l) << K)) << (8 * i);
+    sr |= (run + (run_row<T, HR>(k, one_r) << K)) << (8 * i);
   }
   const uint32_t lo = (uint32_t)((first << 4) & 255);  // the same for every trip of this lane
   const uint32_t lo_l = L.ol[0][lo], lo_r = L.orr[0][lo];
@@ -267,33 +274,44 @@ __device__ void step_quad_kh(const ts_step& st, const LutT<NQ>& L, const uint8_t
     const uint32_t hi = (uint32_t)(o >> 8);
     const uint8_t* pl = lhs + lo_l + hi_off<NQ>(L.ol, hi, nqo);
     const uint8_t* pr = rhs + lo_r + hi_off<NQ>(L.orr, hi, nqo);
-    Run<K + HL> a[4];
-    Run<K + HR> b[4];
+    Run<K + HL> a[G];
+    Run<K + HR> b[G];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) a[g] = load_run<K + HL>(pl + ((g & 1 ? dl[0] : 0u) + (g & 2 ? dl[1] : 0u)));
+    for (int g = 0; g < G; ++g) {
+      uint32_t off = 0;
+#pragma unroll
+      for (int j = 0; j < B; ++j) off += (g >> j) & 1 ? dl[j] : 0u;
+      a[g] = load_run<K + HL>(pl + off);
+    }
     if (!norhs) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) b[g] = load_run<K + HR>(pr + ((g & 1 ? dr[0] : 0u) + (g & 2 ? dr[1] : 0u)));
+      for (int g = 0; g < G; ++g) {
+        uint32_t off = 0;
+#pragma unroll
+        for (int j = 0; j < B; ++j) off += (g >> j) & 1 ? dr[j] : 0u;
+        b[g] = load_run<K + HR>(pr + off);
+      }
     } else {
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
+      for (int g = 0; g < G; ++g)
 #pragma unroll
         for (uint32_t& w : b[g].w) w = ~0u;
     }
     uint32_t res[4];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
+    for (int d = 0; d < 4; ++d) {
       if constexpr (K <= 1) {
-        uint32_t x = quad_bytes<K, HL>(a[g], sl, 0) & quad_bytes<K, HR>(b[g], sr, 0);
-        if constexpr (K == 1) x |= quad_bytes<K, HL>(a[g], sl, 1) & quad_bytes<K, HR>(b[g], sr, 1);
-        res[g] = ((((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x) >> 7) & 0x01010101u;
+        uint32_t x = run_bytes<T>(a, d, sl, 0) & run_bytes<T>(b, d, sr, 0);
+        if constexpr (K == 1) x |= run_bytes<T>(a, d, sl, 1) & run_bytes<T>(b, d, sr, 1);
+        res[d] = ((((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x) >> 7) & 0x01010101u;
       } else {
-        res[g] = 0;
+        res[d] = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          uint32_t x = quad_word<K, HL>(a[g], i, 0, one_l) & quad_word<K, HR>(b[g], i, 0, one_r);
-          if constexpr (K == 3) x |= quad_word<K, HL>(a[g], i, 1, one_l) & quad_word<K, HR>(b[g], i, 1, one_r);
-          res[g] |= (x < 1u ? x : 1u) << (8 * i);
+          const int g = (4 * d + i) >> T, k = i & ((1 << T) - 1);
+          uint32_t x = run_word<T, K, HL>(a[g], k, 0, one_l) & run_word<T, K, HR>(b[g], k, 0, one_r);
+          if constexpr (K == 3) x |= run_word<T, K, HL>(a[g], k, 1, one_l) & run_word<T, K, HR>(b[g], k, 1, one_r);
+          res[d] |= (x < 1u ? x : 1u) << (8 * i);
         }
       }
     }
@@ -301,35 +319,45 @@ __device__ void step_quad_kh(const ts_step& st, const LutT<NQ>& L, const uint8_t
   }
 }
 
-template <int K, int HL, int NQ>
-__device__ __forceinline__ void step_quad_k(const ts_step& st, int hr, const LutT<NQ>& L, const uint8_t* lhs,
+template <int T, int K, int HL, int NQ>
+__device__ __forceinline__ void step_runs_k(const ts_step& st, int hr, const LutT<NQ>& L, const uint8_t* lhs,
                                             const uint8_t* rhs, uint8_t* out, uint64_t first, uint64_t stride) {
-  if (hr == 0) step_quad_kh<K, HL, 0, NQ>(st, L, lhs, rhs, out, first, stride);
-  else if (hr == 1) step_quad_kh<K, HL, 1, NQ>(st, L, lhs, rhs, out, first, stride);
-  else step_quad_kh<K, HL, 2, NQ>(st, L, lhs, rhs, out, first, stride);
+  if (hr == 0) step_runs_kh<T, K, HL, 0, NQ>(st, L, lhs, rhs, out, first, stride);
+  else if (hr == 1) step_runs_kh<T, K, HL, 1, NQ>(st, L, lhs, rhs, out, first, stride);
+  else if constexpr (T == 2) step_runs_kh<T, K, HL, 2, NQ>(st, L, lhs, rhs, out, first, stride);
 }
 
-template <int K, int NQ>
-__device__ __forceinline__ void step_quad_l(const ts_step& st, int hl, int hr, const LutT<NQ>& L, const uint8_t* lhs,
+template <int T, int K, int NQ>
+__device__ __forceinline__ void step_runs_l(const ts_step& st, int hl, int hr, const LutT<NQ>& L, const uint8_t* lhs,
                                             const uint8_t* rhs, uint8_t* out, uint64_t first, uint64_t stride) {
-  if (hl == 0) step_quad_k<K, 0, NQ>(st, hr, L, lhs, rhs, out, first, stride);
-  else if (hl == 1) step_quad_k<K, 1, NQ>(st, hr, L, lhs, rhs, out, first, stride);
-  else step_quad_k<K, 2, NQ>(st, hr, L, lhs, rhs, out, first, stride);
+  if (hl == 0) step_runs_k<T, K, 0, NQ>(st, hr, L, lhs, rhs, out, first, stride);
+  else if (hl == 1) step_runs_k<T, K, 1, NQ>(st, hr, L, lhs, rhs, out, first, stride);
+  else if constexpr (T == 2) step_runs_k<T, K, 2, NQ>(st, hr, L, lhs, rhs, out, first, stride);
 }
 
-// Grid-stride over groups of 16 outputs of a quad_shaped step (first / stride as for
-// step_u8).
+template <int T, int NQ>
+__device__ __forceinline__ void step_runs_t(const ts_step& st, const LutT<NQ>& L, const uint8_t* lhs,
+                                            const uint8_t* rhs, uint8_t* out, uint64_t first, uint64_t stride) {
+  const bool norhs = st.flags & TS_STEP_NORHS;
+  int hl = 0, hr = 0;  // low out bits that each operand holds
+  for (int j = 0; j < T; ++j) {
+    hl += st.o_lpos[j] != TS_NOPOS;
+    hr += !norhs && st.o_rpos[j] != TS_NOPOS;
+  }
+  if (st.sum_rank == 0) step_runs_l<T, 0, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
+  else if (st.sum_rank == 1) step_runs_l<T, 1, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
+  else if (st.sum_rank == 2) step_runs_l<T, 2, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
+  else step_runs_l<T, 3, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
+}
+
+// Grid-stride over groups of 16 outputs of a step with t = run_bits(st) > 0 (first / stride as
+// for step_u8).
 template <int NQ>
-__device__ inline void step_quad(const ts_step& st, const LutT<NQ>& L, const uint8_t* __restrict__ lhs,
+__device__ inline void step_runs(int t, const ts_step& st, const LutT<NQ>& L, const uint8_t* __restrict__ lhs,
                                  const uint8_t* __restrict__ rhs, uint8_t* __restrict__ out, uint64_t first,
                                  uint64_t stride) {
-  const bool norhs = st.flags & TS_STEP_NORHS;
-  const int hl = (st.o_lpos[0] != TS_NOPOS) + (st.o_lpos[1] != TS_NOPOS);
-  const int hr = norhs ? 0 : (st.o_rpos[0] != TS_NOPOS) + (st.o_rpos[1] != TS_NOPOS);
-  if (st.sum_rank == 0) step_quad_l<0, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
-  else if (st.sum_rank == 1) step_quad_l<1, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
-  else if (st.sum_rank == 2) step_quad_l<2, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
-  else step_quad_l<3, NQ>(st, hl, hr, L, lhs, rhs, out, first, stride);
+  if (t == 2) step_runs_t<2, NQ>(st, L, lhs, rhs, out, first, stride);
+  else step_runs_t<1, NQ>(st, L, lhs, rhs, out, first, stride);
 }
 
 // Boolean step over out indices o = first + k * stride (first = block * 256 + tid and

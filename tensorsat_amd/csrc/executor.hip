@@ -38,8 +38,9 @@ __global__ __launch_bounds__(WG) void k_step_u8(const uint8_t* __restrict__ lhs,
   const bool need_c = !(st.flags & TS_STEP_KINNER) && st.sum_rank > 0;
   build_lut(st, L, need_c, threadIdx.x);
   __syncthreads();
-  if (quad_shaped(st))
-    step_quad(st, L, lhs, rhs, out, (uint64_t)blockIdx.x * WG + threadIdx.x, (uint64_t)gridDim.x * WG);
+  const int t = run_bits(st);
+  if (t > 0)
+    step_runs(t, st, L, lhs, rhs, out, (uint64_t)blockIdx.x * WG + threadIdx.x, (uint64_t)gridDim.x * WG);
   else
     step_u8(st, L, lhs, rhs, out, (uint64_t)blockIdx.x * WG + threadIdx.x, (uint64_t)gridDim.x * WG, mode);
 }
@@ -456,8 +457,10 @@ __global__ __launch_bounds__(WG) void k_gang_step(GangStep) {
   }
   build_lut(s_st, L, !kinner && s_st.sum_rank > 0, tid);
   __syncthreads();
-  if (quad_shaped(s_st))
-    step_quad(s_st, L, arena + s_st.lhs_off, rhs, arena + s_st.out_off, (uint64_t)first * WG + tid, (uint64_t)nb * WG);
+  const int t = run_bits(s_st);
+  if (t > 0)
+    step_runs(t, s_st, L, arena + s_st.lhs_off, rhs, arena + s_st.out_off, (uint64_t)first * WG + tid,
+              (uint64_t)nb * WG);
   else
     step_u8(s_st, L, arena + s_st.lhs_off, rhs, arena + s_st.out_off, (uint64_t)first * WG + tid, (uint64_t)nb * WG,
             g.mode);
@@ -1027,12 +1030,12 @@ int make_step(int rl, const int32_t* lw, int rr, const int32_t* rw, int ro, cons
   return TS_OK;
 }
 
-// Workgroups of one step on the step engine.  Short rows (quad_shaped) take 4096 outputs per
+// Workgroups of one step on the step engine.  Short rows (run_bits) take 4096 outputs per
 // trip, and a workgroup's tables cost as much as a few trips, so at most 2048 of them (8 per
 // CU); other steps take 256 outputs or more per trip.
 uint64_t step_blocks(const ts_step& st) {
   const uint64_t n = 1ull << st.out_rank;
-  if (quad_shaped(st)) return std::min<uint64_t>((n + 16 * WG - 1) / (16 * WG), 2048);
+  if (run_bits(st)) return std::min<uint64_t>((n + 16 * WG - 1) / (16 * WG), 2048);
   return (uint64_t)grid_for(n);
 }
 
@@ -1171,7 +1174,7 @@ ContractPlan plan_contract(const ts_step& s0, bool aligned) {
         if (pos[j] != TS_NOPOS && pos[j] != k++) return false;
       return true;
     };
-    if (kinner && quad_shaped(st) && rows_in_order(st.o_lpos) && rows_in_order(st.o_rpos)) return p;
+    if (kinner && run_bits(st) == 2 && rows_in_order(st.o_lpos) && rows_in_order(st.o_rpos)) return p;
     p.kind = PLAN_OUTER;
   } else {
     if (kinner || st.out_rank + nc < TERM_MIN) return p;
