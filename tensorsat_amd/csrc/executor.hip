@@ -1143,7 +1143,14 @@ void regular_layout(ts_step& st, uint8_t* pos, uint8_t* cpos, bool inner, int* p
 //    16 -> 12 us, at 2^18 the two or three launches lose (9 -> 15 us), hence the line;
 //  * otherwise, 2^TERM_MIN or more products: summed bits innermost for the popcount rows of
 //    the step engine.
-// A step already in a layout of the step engine that reads whole runs keeps it.
+// Steps whose summed bits are innermost already (all steps of a compiled program) keep the step
+// engine where it reads whole runs: rows of 16 bytes or more, and shorter ones with their two
+// lowest out bits in order; both the copies and the term walk of k_step_outer lose to it
+// (2^20 outputs, rows of 16 bytes: 11 us, 56 through copies; rows of 4, 2^22 outputs: 14 and
+// 44).  With only the lowest out bit in order the copies are worth it up to half a byte per
+// output (2^24 outputs of single entries, 2^21 entries on either side: 30 us in place, 19
+// copied; 2^23 entries: 23 and 35), with none up to 4 bytes (2^23 outputs over one summed bit,
+// 2^24 entries on either side: 53 and 34; over two, 2^25 entries: 46 and 76).
 constexpr int OUT_MIN = 20, TERM_MIN = 22, DENSE_MIN = 18;
 
 ContractPlan plan_contract(const ts_step& s0, bool aligned) {
@@ -1152,6 +1159,7 @@ ContractPlan plan_contract(const ts_step& s0, bool aligned) {
   p.move_l = p.move_r = false;
   p.at_r = p.bytes = 0;
   p.st = s0;
+  const ContractPlan stay = p;
   ts_step& st = p.st;
   const int nc = st.sum_rank;
   if (!aligned || st.out_rank + nc < DENSE_MIN) return p;
@@ -1168,13 +1176,7 @@ ContractPlan plan_contract(const ts_step& s0, bool aligned) {
     if (kinner) return p;
     p.kind = PLAN_DENSE;
   } else if (nc <= 7 && st.out_rank >= OUT_MIN) {
-    auto rows_in_order = [&](const uint8_t* pos) {  // kept bits right above the summed ones
-      int k = nc;
-      for (int j = 0; j < st.out_rank && k < 6; ++j)
-        if (pos[j] != TS_NOPOS && pos[j] != k++) return false;
-      return true;
-    };
-    if (kinner && run_bits(st) == 2 && rows_in_order(st.o_lpos) && rows_in_order(st.o_rpos)) return p;
+    if (kinner && (nc >= 4 || run_bits(st) == 2)) return p;
     p.kind = PLAN_OUTER;
   } else {
     if (kinner || st.out_rank + nc < TERM_MIN) return p;
@@ -1220,6 +1222,10 @@ ContractPlan plan_contract(const ts_step& s0, bool aligned) {
   const int64_t bl = p.move_l ? (1ll << st.lhs_rank) : 0, br = p.move_r ? (1ll << st.rhs_rank) : 0;
   p.at_r = (bl + 255) & ~255ll;
   p.bytes = p.at_r + br;
+  if (kinner) {  // short rows out of order: what the copies may cost
+    const int64_t outs = 1ll << st.out_rank;
+    if (run_bits(s0) == 1 ? 2 * p.bytes > outs : p.bytes > 4 * outs) return stay;
+  }
   return p;
 }
 

@@ -80,3 +80,39 @@ def test_weight_gradient_scratch_sizes():
     for m, rows in ((-1, 5), (5, -1), (32769, 5)):
         assert L.ts_gnn_wgrad_scratch(m, rows, ctypes.byref(need)) == N.TS_EINVAL
     assert L.ts_gnn_wgrad_scratch(4, 4, None) == N.TS_EINVAL
+
+
+def _contract_scratch(lhs, rhs, out):
+    """Scratch bytes that ts_contract2 can use for these wires (0: it copies no operand)."""
+    from tensorsat_amd import _native as N
+
+    need = N.i64(-1)
+    args = [x for ws in (lhs, rhs, out) for x in (len(ws), N.i32arr(ws))]
+    assert N.load().ts_contract2_scratch(*args, ctypes.byref(need)) == 0
+    return need.value
+
+
+@pytest.mark.parametrize("own", [0, 1, 3])
+@pytest.mark.parametrize("out_bits", [20, 22])
+def test_rows_in_place_are_not_copied(out_bits, own):
+    """Contractions whose summed wires are innermost in both operands: rows of 16 bytes or more,
+    and shorter ones whose two last out wires are each operand's last kept ones."""
+    shared = out_bits - 2 * own
+    kept_l, kept_r = [*range(shared)], [*range(shared)]
+    kept_l[shared // 2 : shared // 2] = range(100, 100 + own)
+    kept_r[shared // 3 : shared // 3] = range(200, 200 + own)
+    out = [*range(100, 100 + own), *range(200, 200 + own), *range(shared)]
+    for k in range(8):
+        if max(len(kept_l), len(kept_r)) + k > 27 or (k >= 6 and own >= 4):
+            continue
+        summed = [*range(300, 300 + k)]
+        for swap in (False, True):  # the wires above the two last ones in any order
+            a, b = list(kept_l), list(kept_r)
+            if swap:
+                a[0], a[3], b[1], b[4] = a[3], a[0], b[4], b[1]
+            assert _contract_scratch(a + summed, b + summed, out) == 0, (k, swap)
+        if 4 <= k:  # any order of the kept wires
+            assert _contract_scratch(kept_l[::-1] + summed, kept_r + summed, out) == 0, k
+        elif own == 0:  # reversed: copied where that costs at most 4 bytes per output
+            size = 2 ** (out_bits + k)
+            assert _contract_scratch(kept_l[::-1] + summed, kept_r[::-1] + summed, out) == (2 * size if k < 2 else 0)
