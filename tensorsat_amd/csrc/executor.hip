@@ -1135,14 +1135,24 @@ void regular_layout(ts_step& st, uint8_t* pos, uint8_t* cpos, bool inner, int* p
 //  * 6 or more summed bits, 4 or more bits held by one operand only on each side, 2^DENSE_MIN
 //    or more products: the summed bits are moved innermost and the matrix cores run the
 //    product.  2^13 x 2^13 by 2^13 x 2^13: 602 ms as byte gathers, 0.50 ms so (0.03 ms of it
-//    the permutation); 2^6 x 2^10 by 2^10 x 2^6: 22 -> 13 us;
+//    the permutation); 2^6 x 2^10 by 2^10 x 2^6: 22 -> 13 us.  2^10 or fewer outputs of 256
+//    or more terms are a few tiles on as many CUs and stay with k_step_dot (2^5 x 2^10 by
+//    2^10 x 2^5: 8 us, 15 us on the matrix cores), and so do 2^11 below 2^16 terms (2^12: 14
+//    to 24 us, 25; from 2^16 on one or the other, by layout);
 //  * at most 7 summed bits (128 terms: both epilogues are "any") and 2^OUT_MIN or more
 //    outputs: k_step_outer, the kept bits of each operand in out order (in runs of 64 bytes;
 //    an operand that has them so is read in place, wherever its summed bits are above).
 //    2^25 and 2^24 entries into 2^26 over one summed bit: 291 -> 50 us.  At 2^20 outputs
 //    16 -> 12 us, at 2^18 the two or three launches lose (9 -> 15 us), hence the line;
 //  * otherwise, 2^TERM_MIN or more products: summed bits innermost for the popcount rows of
-//    the step engine.
+//    the step engine, where the copies pay for themselves.  A gather costs per term: 16 terms
+//    per output are cheap (2^18 outputs: 15 us, 33 us with 2 bytes to copy per product; 2^19
+//    with 0.05: 23 and 13), 32 to 128 lose to copies of up to 1.5 bytes per product (2^19
+//    outputs of 32: 67 us, 33 copied; 2^18 of 128 with 2 bytes: 86 and 123), more always (2^13
+//    of 2^11: 604 and 52).  k_step_dot, a workgroup per output, hides a gather up to 2^15
+//    terms: copies there have to be at most 0.6 bytes per product and the products 2^23 (2^9
+//    outputs of 2^14 terms: 24 -> 13 us; 2^11 of 2^14, a byte per product: 45 us, 85 copied);
+//    longer sums always gain (2^4 of 2^19: 0.69 -> 0.09 ms).
 // Steps whose summed bits are innermost already (all steps of a compiled program) keep the step
 // engine where it reads whole runs: rows of 16 bytes or more, and shorter ones with their two
 // lowest out bits in order; both the copies and the term walk of k_step_outer lose to it
@@ -1173,13 +1183,13 @@ ContractPlan plan_contract(const ts_step& s0, bool aligned) {
   const bool kinner = st.flags & TS_STEP_KINNER;
   const bool dense = nc >= 6 && nm >= 4 && nn >= 4;
   if (dense) {
-    if (kinner) return p;
+    if (kinner || (dot_shaped(st) && (st.out_rank <= 10 || (st.out_rank == 11 && nc < 16)))) return p;
     p.kind = PLAN_DENSE;
   } else if (nc <= 7 && st.out_rank >= OUT_MIN) {
     if (kinner && (nc >= 4 || run_bits(st) == 2)) return p;
     p.kind = PLAN_OUTER;
   } else {
-    if (kinner || st.out_rank + nc < TERM_MIN) return p;
+    if (kinner || nc < 4 || st.out_rank + nc < TERM_MIN) return p;
     p.kind = PLAN_INNER;
   }
   if (p.kind == PLAN_OUTER) {
@@ -1222,6 +1232,15 @@ ContractPlan plan_contract(const ts_step& s0, bool aligned) {
   const int64_t bl = p.move_l ? (1ll << st.lhs_rank) : 0, br = p.move_r ? (1ll << st.rhs_rank) : 0;
   p.at_r = (bl + 255) & ~255ll;
   p.bytes = p.at_r + br;
+  const int64_t products = 1ll << (st.out_rank + nc);
+  if (p.kind == PLAN_INNER) {
+    const bool many = products >= (2ll << TERM_MIN);
+    bool pays = nc >= 8;
+    if (dot_shaped(s0)) pays = nc >= 16 || (many && 5 * p.bytes <= 3 * products);
+    else if (nc == 4) pays = many && 4 * p.bytes <= products;
+    else if (nc < 8) pays = (many || nc > 5) && 2 * p.bytes <= 3 * products;
+    if (!pays) return stay;
+  }
   if (kinner) {  // short rows out of order: what the copies may cost
     const int64_t outs = 1ll << st.out_rank;
     if (run_bits(s0) == 1 ? 2 * p.bytes > outs : p.bytes > 4 * outs) return stay;

@@ -116,3 +116,25 @@ def test_rows_in_place_are_not_copied(out_bits, own):
         elif own == 0:  # reversed: copied where that costs at most 4 bytes per output
             size = 2 ** (out_bits + k)
             assert _contract_scratch(kept_l[::-1] + summed, kept_r[::-1] + summed, out) == (2 * size if k < 2 else 0)
+
+
+def test_small_products_keep_their_gather():
+    """Summed wires outermost in both operands: which products copy them innermost first."""
+    def bytes_for(batch, m, n, k):
+        b, s = [*range(batch)], [*range(300, 300 + k)]
+        l, r = [*range(100, 100 + m)], [*range(200, 200 + n)]
+        return _contract_scratch(s + b + l, s + b + r, b + l + r)
+
+    moved = lambda batch, m, n, k: 2 ** (batch + m + k) + 2 ** (batch + n + k)
+    # matrix cores: not for 2^10 or fewer outputs of 256 or more terms, 2^11 of less than 2^16
+    for shape, copies in (((0, 4, 4, 12), False), ((0, 5, 5, 10), False), ((2, 4, 4, 8), False), ((0, 5, 6, 12), False),
+                          ((0, 5, 6, 16), True), ((0, 6, 6, 8), True), ((4, 4, 4, 6), True), ((0, 6, 6, 6), True)):
+        assert bytes_for(*shape) == (moved(*shape) if copies else 0), shape
+    # a workgroup per output: long sums, or half a byte to copy per product and 2^23 of them
+    for shape, copies in (((4, 3, 3, 12), False), ((8, 0, 1, 13), False), ((12, 0, 0, 11), False), ((2, 2, 5, 14), True),
+                          ((0, 2, 2, 16), False), ((1, 2, 3, 16), True), ((2, 0, 2, 18), True)):
+        assert bytes_for(*shape) == (moved(*shape) if copies else 0), shape
+    # rows of the step engine
+    for shape, copies in (((18, 0, 0, 4), False), ((14, 3, 1, 4), False), ((8, 3, 8, 4), True), ((16, 1, 0, 5), False),
+                          ((16, 2, 1, 5), True), ((18, 0, 0, 7), False), ((16, 1, 1, 7), True), ((10, 0, 3, 11), True)):
+        assert bytes_for(*shape) == (moved(*shape) if copies else 0), shape
