@@ -363,15 +363,19 @@ struct GangStep {
   uint8_t* arena[GANG];
   uint32_t blk[GANG + 1];
   uint32_t pk[GANG];
-  uint8_t kind[GANG];
+  uint32_t kind[GANG];
   int32_t n, mode;
 };
+// Per-job entries of kernel arguments are dwords or pointers, never bytes: from kind[j] as a byte
+// the compiler formed the address of pk[j] as (arguments + j) + 3 j, and a scalar load drops
+// the low two bits of either part -- with more than one job it read another job's offset.
+static_assert(sizeof(GangStep::kind) == 4 * GANG, "dword entries");
 
 struct GangPack {  // pack tasks: rows of 2^k bytes -> 2^k-bit masks (k = 4..10)
   const uint8_t* src[2 * GANG];
   uint8_t* dst[2 * GANG];
   uint32_t rows[2 * GANG];
-  uint8_t k[2 * GANG];
+  uint32_t k[2 * GANG];  // dwords: see GangStep
 };
 
 struct GangCopy {
@@ -419,9 +423,7 @@ __global__ __launch_bounds__(WG) void k_gang_step(GangStep) {
   const GangStep& g = kernarg<GangStep>();
   const uint32_t b = blockIdx.x;
   const int tid = threadIdx.x;
-  // The job of this block: the last one that starts at or below it, by halving.  Scalar loads
-  // only: a wave-wide ballot here went wrong where one lane alone uses the job (below: it took
-  // another job's mask offset).
+  // The job of this block: the last one that starts at or below it, by halving.
   int j = 0;
   for (int h = GANG / 2; h > 0; h >>= 1)
     if (j + h < g.n && g.blk[j + h] <= b) j += h;
@@ -1897,11 +1899,11 @@ int ts_program_run_gang(const ts_job* jobs, int32_t count, const ts_step* steps,
         pkd.src[npk] = ar + st.lhs_off;
         pkd.dst[npk] = ar + pk;
         pkd.rows[npk] = lrows;
-        pkd.k[npk++] = (uint8_t)k;
+        pkd.k[npk++] = (uint32_t)k;
         pkd.src[npk] = ar + st.rhs_off;
         pkd.dst[npk] = ar + pk + packed_rhs_at(st);
         pkd.rows[npk] = rrows;
-        pkd.k[npk++] = (uint8_t)k;
+        pkd.k[npk++] = (uint32_t)k;
         pk_rows = std::max(pk_rows, std::max(lrows, rrows));
         t.kind[nt] = 2;
         t.pk[nt] = (uint32_t)pk;
