@@ -116,6 +116,20 @@ __host__ __device__ inline uint64_t packed_bytes(const ts_step& st) {
   return packed_rhs_at(st) + (1ull << (st.rhs_rank - 3));
 }
 
+// The record of the same step on rows packed at arena offset pk (lhs, then rhs): what the
+// kernel runs, and what the host sizes its launch by.
+__host__ __device__ inline void pack_record(ts_step& st, uint32_t pk) {
+  st.rhs_off = pk + packed_rhs_at(st);
+  st.lhs_off = pk;
+  st.lhs_rank -= 3;
+  st.rhs_rank -= 3;
+  st.sum_rank -= 3;
+  for (int q = 0; q < st.out_rank; ++q) {
+    if (st.o_lpos[q] != TS_NOPOS) st.o_lpos[q] -= 3;
+    if (st.o_rpos[q] != TS_NOPOS) st.o_rpos[q] -= 3;
+  }
+}
+
 // Rule shared by the host dispatch: at least 2^8 terms per output, at most 2^12 outputs,
 // summed bits innermost (16-byte runs) or not.
 inline bool dot_shaped(const ts_step& st) { return st.sum_rank >= 8 && st.out_rank <= 12; }
@@ -431,18 +445,7 @@ __global__ __launch_bounds__(WG) void k_gang_step(GangStep) {
     reinterpret_cast<uint4*>(&s_st)[tid] = reinterpret_cast<const uint4*>(g.rec[j])[tid];
   __syncthreads();
   if (g.kind[j] == 2) {  // the same step on the packed rows
-    if (tid == 0) {
-      const uint32_t pk = g.pk[j];
-      s_st.rhs_off = pk + packed_rhs_at(s_st);
-      s_st.lhs_off = pk;
-      s_st.lhs_rank -= 3;
-      s_st.rhs_rank -= 3;
-      s_st.sum_rank -= 3;
-      for (int q = 0; q < s_st.out_rank; ++q) {
-        if (s_st.o_lpos[q] != TS_NOPOS) s_st.o_lpos[q] -= 3;
-        if (s_st.o_rpos[q] != TS_NOPOS) s_st.o_rpos[q] -= 3;
-      }
-    }
+    if (tid == 0) pack_record(s_st, g.pk[j]);
     __syncthreads();
   }
   uint8_t* arena = g.arena[j];
@@ -1908,7 +1911,9 @@ int ts_program_run_gang(const ts_job* jobs, int32_t count, const ts_step* steps,
         t.kind[nt] = 2;
         t.pk[nt] = (uint32_t)pk;
       }
-      const uint64_t b = t.kind[nt] == 1 ? (1ull << st.out_rank) : step_blocks(st);
+      ts_step run = st;  // as its blocks run it: packed rows of up to 8 bytes are short rows
+      if (t.kind[nt] == 2) pack_record(run, t.pk[nt]);
+      const uint64_t b = t.kind[nt] == 1 ? (1ull << st.out_rank) : step_blocks(run);
       wants.push_back(b);
       if (t.kind[nt] != 1) want += b;
       if (++nt == GANG) {
