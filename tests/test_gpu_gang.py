@@ -164,3 +164,99 @@ def test_gang_packed_rows_of_different_jobs():
                 o, n = j * stride + int(dp.jobs_host["result_off"][j]), 1 << int(dp.jobs_host["result_rank"][j])
                 print(f"{mode} small {small_bits} job {j}: step {last[j]}, {n} outputs", flush=True)
                 assert torch.equal(arena[o : o + n], want[j])
+
+
+def _dense_program(rng, shapes):
+    """One job per (m, n, b, k) in ``shapes``: a single dense record over random leaves, all
+    records of a shape alike."""
+    steps, jobs, leaves, layouts = [], [], [], {}
+    for i, (m, n, b, k) in enumerate(shapes):
+        ro = m + n + b
+        side = layouts.setdefault((m, n, b, k), rng.permutation(np.repeat([0, 1, 2], [m, n, b])))
+        st, rec = np.zeros(1, PG.STEP_DTYPE), np.zeros(1, PG.JOB_DTYPE)
+        for name, other in (("o_lpos", 1), ("o_rpos", 0)):
+            st[name] = PG.NOPOS
+            st[name][0, :ro][side != other] = k + np.arange((side != other).sum())
+        for name in ("c_lpos", "c_rpos"):
+            st[name] = PG.NOPOS
+            st[name][0, :k] = range(k)
+        lsz, rsz = 1 << (k + m + b), 1 << (k + n + b)
+        st["lhs_rank"], st["rhs_rank"], st["out_rank"], st["sum_rank"] = k + m + b, k + n + b, ro, k
+        st["rhs_off"], st["out_off"], st["flags"] = lsz, lsz + rsz, PG.STEP_KINNER
+        rec["step_begin"], rec["num_steps"], rec["instance"] = i, 1, i
+        rec["leaf_begin"], rec["num_leaf_bytes"] = sum(x.size for x in leaves), lsz + rsz
+        rec["result_off"], rec["result_rank"], rec["max_rank"] = lsz + rsz, ro, max(ro, k + b + max(m, n))
+        rec["arena_elems"] = lsz + rsz + (1 << ro)
+        steps.append(st)
+        jobs.append(rec)
+        leaves.append((rng.random(lsz + rsz) < rng.choice([0.02, 0.1, 1.0])).astype(np.uint8))
+    prog = PG.Program(np.concatenate(jobs), np.concatenate(steps), np.concatenate(leaves),
+                      np.zeros((len(shapes), PG.NSTAT), np.int64), {})
+    PG.validate(prog)
+    return prog
+
+
+@pytest.mark.parametrize("mode", ["GT0", "MOD256"])
+def test_gang_of_dense_steps(mode):
+    """Matrix-core steps of several jobs in one launch: more jobs than one launch holds, changes
+    of shape, two shapes in turn, and jobs without such a step between them."""
+    import torch
+
+    from tensorsat_amd.executor import DeviceProgram, gang_stride, run_gang, run_job
+
+    a, b, c = (5, 4, 1, 8), (4, 6, 0, 6), (6, 5, 2, 9)
+    slow = (2, 3, 4, 6)  # too few bits on either side
+    shapes = [a] * 67 + [b] * 3 + [c, a, c, a, a] + [slow, b, slow, slow, b, c, c]
+    prog = _dense_program(np.random.default_rng(12), shapes)
+    dp = DeviceProgram(prog)
+    stride, n = gang_stride(dp), len(shapes)
+    arena = torch.full((n * stride,), 255, dtype=torch.uint8, device="cuda")
+    flags = run_gang(dp, 0, n, mode, arena=arena, small_bits=0).cpu().numpy()
+    seen = set()
+    for j in range(n):
+        print(f"{mode} job {j} shape {shapes[j]}", flush=True)
+        want = OX.run_job(prog, j, mode)[0].reshape(-1)
+        at = j * stride + int(prog.jobs["result_off"][j])
+        np.testing.assert_array_equal(arena[at : at + want.size].cpu().numpy(), want)
+        np.testing.assert_array_equal(run_job(dp, j, mode)[0].cpu().numpy().reshape(-1), want)
+        assert flags[j] == int(want.any())
+        seen.add(want.tobytes())
+    assert len(seen) > n // 2  # the jobs' results differ
+
+
+@pytest.mark.parametrize("mode", ["GT0", "MOD256"])
+def test_staged_runs_at_the_limit(mode):
+    """Runs of small steps whose tensors end at the last entry that is staged in LDS (65536), one
+    piece below and one above, beside jobs that end far below."""
+    import torch
+
+    from tensorsat_amd.executor import DeviceProgram, gang_stride, run_gang
+
+    parts, want = [], []
+    for i, end in enumerate((65536, None, 65520, 65552, None, 65536)):
+        w = CNFInstance.random(3, 10, 35, rng=60 + i)
+        d = (w.inputs("_" * 10) >> w.diagram()).flatten()
+        p = PG.compile_network(d.wiring, list(d.blocks), PG.elim(d.wiring, trials=1))
+        assert len(p.steps) >= 65
+        shift = 0 if end is None else end - int(p.jobs["arena_elems"][0])
+        for name in ("lhs_off", "rhs_off", "out_off"):
+            p.steps[name] += shift
+        for name in ("num_leaf_bytes", "result_off", "arena_elems"):
+            p.jobs[name] += shift
+        top = max(int(p.steps["out_off"][k]) + (1 << int(p.steps["out_rank"][k])) for k in range(len(p.steps)))
+        p.leaves = np.concatenate([np.full(shift, 3, np.uint8), p.leaves])
+        assert end is None or top == end
+        parts.append(p)
+        want.append(OX.run_job(p, 0, mode)[0].reshape(-1))
+    prog = PG.concat(parts, [np.array([i]) for i in range(6)], 6)
+    PG.validate(prog)
+    dp = DeviceProgram(prog)
+    stride = gang_stride(dp)
+    for small_bits in (12, 9):
+        arena = torch.full((6 * stride,), 255, dtype=torch.uint8, device="cuda")
+        flags = run_gang(dp, 0, 6, mode, arena=arena, small_bits=small_bits).cpu().numpy()
+        for j in range(6):
+            at = j * stride + int(prog.jobs["result_off"][j])
+            print(f"{mode} small {small_bits} job {j}", flush=True)
+            np.testing.assert_array_equal(arena[at : at + want[j].size].cpu().numpy(), want[j])
+            assert flags[j] == int(want[j].any())

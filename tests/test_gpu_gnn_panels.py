@@ -119,3 +119,50 @@ def test_relu_backward(rows):
     np.testing.assert_array_equal(dz.float().cpu().numpy(),
                                   torch.from_numpy(want.astype(np.float32)).to(torch.bfloat16).float().numpy())
     _close(db, want.sum(0) + 0.25, np.abs(want).sum(0) + 1, rows + 2)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("F", [1, 64, 65, 100, 128])
+@pytest.mark.parametrize("rows", [1, 3, 4, 5, 2049])
+def test_head(rows, F, masked):
+    """Outputs, loss and gradients of the scalar head: u = 2^-24 per operation, carried through
+    y -> d = y - t -> g = 2 m d / n to the sums."""
+    import torch
+
+    from tensorsat_amd import _native as N_
+
+    rng = np.random.default_rng([rows, F, masked])
+    ldh = F + 5
+    h = torch.relu(_bf(rng, rows, ldh))
+    w, b, t = (torch.from_numpy(rng.standard_normal(n).astype(np.float32)).cuda() for n in (F, 1, rows))
+    m = torch.from_numpy((rng.random(rows) < 0.7).astype(np.float32)).cuda() if masked else None
+    inv = float(np.float32(1.0 / rows))
+    y, dh = torch.full((rows + 1,), 9.0, device="cuda"), torch.full((rows * F + 1,), 9.0, device="cuda")
+    dw, db, loss = (torch.full((n,), 0.5, device="cuda") for n in (F, 1, 1))
+    print(f"rows {rows} F {F} mask {masked}", flush=True)
+    base = (N_.dptr(h), ldh, rows, N_.dptr(w), N_.dptr(b))
+    N_.check(N_.lib().ts_gnn_head(*base, None, None, 0.0, N_.dptr(y), None, None, None, None, F, 0, N_.stream_ptr()), "head")
+    infer = y.clone()
+    N_.check(N_.lib().ts_gnn_head(*base, N_.dptr(t), N_.dptr(m) if masked else None, inv, N_.dptr(y), N_.dptr(loss),
+                                  N_.dptr(dh), N_.dptr(dw), N_.dptr(db), F, 1, N_.stream_ptr()), "head")
+    assert torch.equal(y, infer) and float(y[rows]) == 9.0 and float(dh[rows * F]) == 9.0
+    h64, w64, b64, t64 = (x.double().cpu().numpy() for x in (h[:, :F], w, b, t))
+    m64 = m.double().cpu().numpy() if masked else np.ones(rows)
+    u = 2.0**-24
+
+    def close(got, want, bound):
+        err = np.abs(got.double().cpu().numpy().reshape(want.shape) - want)
+        assert (err <= bound + 1e-30).all(), (err / (bound + 1e-30)).max()
+
+    y64 = h64 @ w64 + b64
+    ey = (F + 1) * u * (np.abs(h64) @ np.abs(w64) + np.abs(b64))
+    close(y[:rows], y64, ey)
+    d = y64 - t64
+    ed = ey + u * np.abs(d)
+    g, eg = 2 * m64 * d * inv, 2 * m64 * inv * (ed + 4 * u * np.abs(d))
+    close(dh[: rows * F], g[:, None] * w64, eg[:, None] * np.abs(w64) + u * np.abs(g[:, None] * w64))
+    many = (rows + 4) * u  # the rows' sums, in any order, and the value they are added to
+    close(dw, g @ h64 + 0.5, eg @ np.abs(h64) + many * (np.abs(g) @ np.abs(h64) + 0.5))
+    close(db, np.array([g.sum() + 0.5]), eg.sum() + many * (np.abs(g).sum() + 0.5))
+    sq = m64 * d * d * inv
+    close(loss, np.array([sq.sum() + 0.5]), (2 * m64 * np.abs(d) * inv * ed).sum() + many * (sq.sum() + 0.5) + 4 * u * sq.sum())

@@ -156,6 +156,42 @@ def test_small_trees_match_the_walk_and_the_oracle(mode):
                                               PlannedContraction(OracleRel, d.wiring).contract(d).tensor)
 
 
+def _wide_tree(rng):
+    """28672 leaf entries at most and a result of 2^15: an arena of 65056 of 65536 entries."""
+    ws = [[8, 3], [9, 0], [11, 0, 12, 6, 4, 8, 15, 10], [1, 9, 4, 14, 13, 7, 8, 0, 6, 15, 5, 3, 10],
+          [7, 13, 6, 0, 10, 15, 12, 2, 5, 11, 8], [13, 14, 1, 7, 10, 11, 9, 4]]
+    out = [13, 9, 4, 1, 3, 14, 0, 7, 6, 11, 15, 10, 5, 8, 12]
+    return Diagram(Wiring([2] * 16, ws, out), [(rng.random((2,) * len(s)) < 0.9).astype(np.uint8) for s in ws])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["GT0", "MOD256"])
+def test_largest_arenas(mode):
+    """Up to the 65536 entries of LDS that a job may take; one more is refused."""
+    import torch
+
+    from tensorsat_amd import _native as N
+    from tensorsat_amd.rel import DeviceRel
+
+    d = _wide_tree(np.random.default_rng(8))
+    c = PlannedContraction(DeviceRel, d.wiring)
+    want = _walk(d.wiring, c.tree, d.blocks, mode)
+    with DeviceRel.mode_scope(mode):
+        np.testing.assert_array_equal(c.contract(d).tensor.reshape(-1), want)
+    small = c._small
+    assert small is not None and int(small.prog.jobs["arena_elems"][0]) > 65000
+    steps, bits = torch.from_numpy(small.prog.steps.view(np.uint8)).cuda(), small.leaf_bits(d.blocks)
+    for elems in (65536, 65537):
+        job = small.prog.jobs.copy()
+        job["arena_elems"] = elems
+        res = torch.full((1 << 15,), 7, dtype=torch.uint8, device="cuda")
+        print(f"{mode}: {elems} arena entries", flush=True)
+        rc = N.lib().ts_program_run_small(N.host_ptr(job), N.host_ptr(small.prog.steps), N.dptr(steps), N.host_ptr(bits),
+                                          N.dptr(res), N.MODES[mode], N.stream_ptr())
+        assert rc == (0 if elems == 65536 else N.TS_EUNSUPPORTED)
+        np.testing.assert_array_equal(res.cpu().numpy(), want if rc == 0 else np.full(1 << 15, 7))
+
+
 @pytest.mark.gpu
 def test_device_blocks_and_other_streams():
     import torch
