@@ -24,7 +24,10 @@ TS_EHIP = -5
 BATCH_LDS_MAX = 65536
 SMALL_ARENA = 65536  # TS_SMALL_ARENA
 SMALL_LEAVES = 28672  # leaf entries of a job run in one launch
-SCRATCH_MIN_BITS = 12  # contractions without a tensor of this rank never take scratch memory
+# Contractions below all three never take scratch memory (the lines of the native rule).
+SCRATCH_BITS = 22  # bits of products
+SCRATCH_OUT_BITS = 20  # bits of outputs
+SCRATCH_DENSE_BITS = 18  # bits of products, with 6 or more summed
 BATCH_SEGMENTS = 8  # queue counters per dispatch (TS_BATCH_SEGMENTS)
 BATCH_COUNTER_STRIDE = 64  # int32s between queue counters (TS_BATCH_COUNTER_STRIDE)
 BATCH_COUNTER_INTS = BATCH_SEGMENTS * BATCH_COUNTER_STRIDE

@@ -363,17 +363,22 @@ class DeviceRel:
         res = _empty(1 << len(bo))
         L = N.lib()
         wl, wr, wo = N.i32arr(bl), N.i32arr(br), N.i32arr(bo)
+        out_bits, products = len(bo), len(ids)
+        args = (N.dptr(lhs._data), len(bl), wl, N.dptr(rhs._data), len(br), wr, N.dptr(res), len(bo), wo,
+                N.MODES[DeviceRel._mode])
         # Operands of large contractions are permuted into scratch memory where their wire
         # order needs it; it goes back to the allocator on this stream after the launches.
-        need = N.i64(0)
-        if max(len(bl), len(br), len(bo)) >= N.SCRATCH_MIN_BITS:
+        # Smaller ones never take any, and asking would be a twentieth of their host time.
+        if products >= N.SCRATCH_BITS or out_bits >= N.SCRATCH_OUT_BITS or \
+                (products >= N.SCRATCH_DENSE_BITS and products - out_bits >= 6):
+            need = N.i64(0)
             N.check(L.ts_contract2_scratch(len(bl), wl, len(br), wr, len(bo), wo, ctypes.byref(need)),
                     "ts_contract2_scratch")
-        scratch = _empty(need.value) if need.value else None
-        N.check(L.ts_contract2_into(
-            N.dptr(lhs._data), len(bl), wl, N.dptr(rhs._data), len(br), wr, N.dptr(res), len(bo), wo,
-            N.MODES[DeviceRel._mode], N.dptr(scratch) if need.value else None, need.value, N.stream_ptr()),
-            "ts_contract2")
+            scratch = _empty(need.value) if need.value else None
+            N.check(L.ts_contract2_into(*args, None if scratch is None else N.dptr(scratch), need.value,
+                                        N.stream_ptr()), "ts_contract2")
+        else:
+            N.check(L.ts_contract2(*args, N.stream_ptr()), "ts_contract2")
         box = DeviceRel._new(res, out_shape)
         if len(uniq_out) != len(out_wires):
             box = box._rewire([uniq_out.index(w) for w in out_wires])

@@ -138,3 +138,26 @@ def test_small_products_keep_their_gather():
     for shape, copies in (((18, 0, 0, 4), False), ((14, 3, 1, 4), False), ((8, 3, 8, 4), True), ((16, 1, 0, 5), False),
                           ((16, 2, 1, 5), True), ((18, 0, 0, 7), False), ((16, 1, 1, 7), True), ((10, 0, 3, 11), True)):
         assert bytes_for(*shape) == (moved(*shape) if copies else 0), shape
+
+
+def test_no_scratch_below_the_lines_that_callers_ask_from():
+    """The native rule and the bits from which it is asked agree: random wires just below."""
+    import random
+
+    from tensorsat_amd import _native as N
+
+    rng, asked = random.Random(1), 0
+    for _ in range(4000):
+        batch, m, n, k = rng.randint(0, 19), rng.randint(0, 10), rng.randint(0, 10), rng.randint(0, 16)
+        out, products = batch + m + n, batch + m + n + k
+        if batch + max(m, n) + k > 27 or not 14 <= products <= 24:
+            continue
+        lhs = [*range(batch), *range(100, 100 + m), *range(300, 300 + k)]
+        rhs = [*range(batch), *range(200, 200 + n), *range(300, 300 + k)]
+        res = [*range(batch), *range(100, 100 + m), *range(200, 200 + n)]
+        for ws in (lhs, rhs, res):
+            rng.shuffle(ws)
+        ask = products >= N.SCRATCH_BITS or out >= N.SCRATCH_OUT_BITS or (products >= N.SCRATCH_DENSE_BITS and k >= 6)
+        asked += ask
+        assert ask or _contract_scratch(lhs, rhs, res) == 0, (lhs, rhs, res)
+    assert 200 < asked < 3000
