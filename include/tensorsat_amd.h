@@ -166,15 +166,16 @@ int ts_program_run_small(const ts_job* job, const ts_step* steps, const ts_step*
  * on the host), job g in arena + g * arena_stride (arena_stride a multiple of 256 and at
  * least every job's arena_elems): the jobs advance phase by phase -- phase p is each
  * job's p-th segment, a run of small steps or one large step -- with one launch per
- * phase for all the runs (one workgroup per job), one for the large steps (blocks shared
- * out among the jobs; steps with few outputs and many summed terms get one workgroup
- * per output) and one per MFMA-routed step.  Where the stride leaves room after a job's
+ * phase for all the runs (one workgroup per job; longer runs whose tensors lie in the first
+ * 64 KiB of the arena work on a copy in LDS), one for the large steps (blocks shared out
+ * among the jobs; steps with few outputs and many summed terms get one workgroup per
+ * output) and one per shape of MFMA-routed step for up to 64 jobs.  Where the stride leaves room after a job's
  * arena (rounded up to 256 bytes), a large step whose rows of 2^4..2^10 bytes (summed
  * wires innermost in both operands) are read by many outputs has both operands' rows
  * packed into bit masks there first and runs on the masks (the same counts).  results[g]
- * (device) = 1 if any entry of job g's result is nonzero, else 0.  The slices of a sliced tree (cotengra.py:100-128) and
- * the cubes of one instance are gangs: their small steps, one workgroup each when run
- * alone, share the device.  Enqueued on `stream`; no allocation. */
+ * (device) = 1 if any entry of job g's result is nonzero, else 0.  The slices of a sliced
+ * tree (cotengra.py:100-128) and the cubes of one instance are gangs: their small steps, one
+ * workgroup each when run alone, share the device.  Enqueued on `stream`; no allocation. */
 int ts_program_run_gang(const ts_job* jobs_host, int32_t count, const ts_step* steps_host,
                         const ts_step* steps_dev, const uint8_t* leaves_dev, uint8_t* arena, int64_t arena_stride,
                         uint8_t* results, int32_t mode, int32_t small_bits, ts_stream stream);
