@@ -191,82 +191,123 @@ extern "C" int tsc_packetize(ts_job* jobs, int64_t num_jobs, ts_step* steps, int
 
 namespace {
 
-struct Held {  // arena entries [off, off + len) as the last write to them left them
-  uint32_t off, len;
-  int step, bound;    // step: the one that wrote them
-  int8_t rank, kind;  // rank -1: what is left of a tensor, a part of it overwritten
-  uint64_t end() const { return (uint64_t)off + len; }
-};
+// The tensors of one job: step outputs (tensor i: step i) and, after them, leaves (one per
+// read).  Scratch of count_widths_job, kept from job to job.
+struct JobTensors {
+  struct Slot {  // open addressing: the last step that wrote at an arena offset
+    uint32_t off;
+    int step;
+  };
+  std::vector<Slot> table;
+  std::vector<int> bound, last;           // per step: summed bits below; last step that reads it (-1: none)
+  std::vector<int> reads;                 // two per step: tensor or -1
+  std::vector<int> leaf_off, leaf_end;    // leaves
+  std::vector<int> lo, hi;                // entries [lo, hi) of the tensors still to be read
+  std::vector<int> id, at;                // their tensors, and where a tensor is among them
 
-// Written entries of one job's arena, sorted and disjoint.
-struct HeldSet {
-  std::vector<Held> v;
-
-  size_t first_past(uint64_t off) const {  // first entry that ends after off
-    return std::upper_bound(v.begin(), v.end(), off, [](uint64_t o, const Held& h) { return o < h.end(); }) - v.begin();
+  Slot& slot(uint32_t off) {
+    const size_t mask = table.size() - 1;
+    size_t h = (off * 0x9e3779b1u) & mask;
+    while (table[h].off != UINT32_MAX && table[h].off != off) h = (h + 1) & mask;
+    return table[h];
   }
-  // The tensor that fills [off, off + 2^rank); *touched: anything was written there.
-  const Held* find(uint64_t off, int rank, bool* touched) const {
-    const size_t i = first_past(off);
-    *touched = i < v.size() && v[i].off < off + (1ull << rank);
-    return *touched && v[i].off == off && v[i].rank == rank ? &v[i] : nullptr;
+  void add(int t, int off, int end) {
+    at[t] = (int)id.size();
+    id.push_back(t);
+    lo.push_back(off);
+    hi.push_back(end);
   }
-  void write(const Held& h) {
-    const size_t i = first_past(h.off);
-    size_t j = i;
-    while (j < v.size() && v[j].off < h.end()) ++j;
-    Held keep[3];
-    size_t n = 0;
-    if (i < j && v[i].off < h.off) keep[n++] = Held{v[i].off, h.off - v[i].off, 0, 0, -1, 0};
-    keep[n++] = h;
-    if (i < j && v[j - 1].end() > h.end())
-      keep[n++] = Held{(uint32_t)h.end(), (uint32_t)(v[j - 1].end() - h.end()), 0, 0, -1, 0};
-    const size_t m = std::min(n, j - i);  // overwritten in place
-    std::copy(keep, keep + m, v.begin() + (long)i);
-    if (n > m) v.insert(v.begin() + (long)(i + m), keep + m, keep + n);
-    else v.erase(v.begin() + (long)(i + m), v.begin() + (long)j);
+  void drop(int t) {
+    const int k = at[t];
+    at[id.back()] = k;
+    id[k] = id.back();
+    lo[k] = lo.back();
+    hi[k] = hi.back();
+    id.pop_back();
+    lo.pop_back();
+    hi.pop_back();
+  }
+  bool any(int off, int end) const {  // does any of them lie in [off, end)?
+    const int *l = lo.data(), *h = hi.data();
+    int hit = 0;
+    for (int k = 0, m = (int)lo.size(); k < m; ++k) hit |= (l[k] < end) & (h[k] > off);
+    return hit;
   }
 };
 
 // One job's tags; false if an operand or the result is not a whole tensor written before (or
-// leaf entries that no step wrote to).
-bool count_widths_job(const ts_job& job, ts_step* st, const uint8_t* leaves, HeldSet& held,
+// leaf entries that no step wrote to): first who reads what, by offset, then whether any write
+// overlaps a tensor that is still to be read.
+bool count_widths_job(const ts_job& job, const ts_step* st, const uint8_t* leaves, JobTensors& T,
                       std::vector<uint8_t>& tags) {
   const int n = job.num_steps;
-  held.v.clear();
+  size_t cap = 64;
+  while (cap < 4u * (size_t)(n + 1)) cap *= 2;
+  T.table.assign(cap, JobTensors::Slot{UINT32_MAX, 0});
+  T.bound.assign(n, 0);
+  T.last.assign(n, -1);
+  T.reads.assign(2 * (size_t)n, -1);
+  T.leaf_off.clear();
+  T.leaf_end.clear();
+  tags.assign(n, 0);
   int leaf_bits = 0;
   for (int32_t i = 0; i < job.num_leaf_bytes; ++i)
     if (leaves[job.leaf_begin + i] > 1) leaf_bits = 8;
-  tags.assign(n, 0);
-  bool touched;
+  auto leaf = [&](uint32_t off, int rank) {
+    T.leaf_off.push_back((int)off);
+    T.leaf_end.push_back((int)(off + (1u << rank)));
+    return n + (int)T.leaf_off.size() - 1;
+  };
+  if (job.arena_elems > INT32_MAX) return false;
   for (int i = 0; i < n; ++i) {
     const ts_step& s = st[i];
     int bound = s.sum_rank, kinds[2] = {0, 0};
     for (int side = 0; side < ((s.flags & TS_STEP_NORHS) ? 1 : 2); ++side) {
       const uint32_t off = side ? s.rhs_off : s.lhs_off;
       const int rank = side ? s.rhs_rank : s.lhs_rank;
-      const Held* h = held.find(off, rank, &touched);
-      if (h) {
-        bound += h->bound;
-        kinds[side] = h->kind;
+      const JobTensors::Slot& h = T.slot(off);
+      if (h.off == off) {
+        if (st[h.step].out_rank != rank) return false;
+        bound += T.bound[h.step];
+        kinds[side] = (tags[h.step] & TS_COUNT_OUT32) ? 1 : 0;
+        T.last[h.step] = i;
+        T.reads[2 * i + side] = h.step;
       } else {
-        if (touched || (uint64_t)off + (1ull << rank) > (uint64_t)job.num_leaf_bytes) return false;
+        if ((uint64_t)off + (1ull << rank) > (uint64_t)job.num_leaf_bytes) return false;
         bound += leaf_bits;
         kinds[side] = 2;  // leaves are copied as uint64
+        T.reads[2 * i + side] = leaf(off, rank);
       }
     }
     // values up to 2^bound: uint32 holds 2^31, uint64 holds 2^63
     const bool narrow = bound <= 31, exact = bound <= 63;
     tags[i] = (uint8_t)(kinds[0] | (kinds[1] << 2) | (narrow ? TS_COUNT_OUT32 : 0) | (exact ? TS_COUNT_EXACT : 0));
-    held.write(Held{s.out_off, 1u << s.out_rank, i, bound, (int8_t)s.out_rank, (int8_t)(narrow ? 1 : 0)});
+    T.bound[i] = bound;
+    T.slot(s.out_off) = JobTensors::Slot{s.out_off, i};
   }
-  // The result is read as uint64; it is the last tensor at its place, so no step reads it.
-  const Held* res = held.find((uint64_t)job.result_off, job.result_rank, &touched);
-  if (touched && !res) return false;
-  if (res) {
-    for (int i = res->step + 1; i < n; ++i)
-      if (st[i].lhs_off == res->off || (!(st[i].flags & TS_STEP_NORHS) && st[i].rhs_off == res->off)) return false;
-    tags[res->step] &= (uint8_t)~TS_COUNT_OUT32;
+  // The result is read as uint64: by no step, and after all of them.
+  const JobTensors::Slot& res = T.slot((uint32_t)job.result_off);
+  if (res.off == (uint32_t)job.result_off) {
+    if (st[res.step].out_rank != job.result_rank || T.last[res.step] >= 0) return false;
+    tags[res.step] &= (uint8_t)~TS_COUNT_OUT32;
+    T.last[res.step] = n;
+  } else {
+    leaf((uint32_t)job.result_off, job.result_rank);
+  }
+  T.lo.clear();
+  T.hi.clear();
+  T.id.clear();
+  T.at.resize((size_t)n + T.leaf_off.size());
+  for (size_t k = 0; k < T.leaf_off.size(); ++k) T.add(n + (int)k, T.leaf_off[k], T.leaf_end[k]);
+  for (int i = 0; i < n; ++i) {
+    for (int side = 0; side < 2; ++side) {
+      const int t = T.reads[2 * i + side];
+      if (t >= n || (t >= 0 && T.last[t] == i && !(side && t == T.reads[2 * i]))) T.drop(t);
+    }
+    if ((uint64_t)st[i].out_off + (1ull << st[i].out_rank) > (uint64_t)job.arena_elems) return false;
+    const int off = (int)st[i].out_off, end = off + (1 << st[i].out_rank);
+    if (T.any(off, end)) return false;
+    if (T.last[i] > i) T.add(i, off, end);
   }
   return true;
 }
@@ -296,11 +337,11 @@ extern "C" int tsc_count_widths(const ts_job* jobs, int64_t num_jobs, ts_step* s
   int nt = threads > 0 ? threads : (int)std::max(1u, std::thread::hardware_concurrency());
   nt = (int)std::max<int64_t>(1, std::min<int64_t>(nt, num_jobs / 64 + 1));
   auto work = [&](int t) {
-    HeldSet held;
+    JobTensors tensors;
     std::vector<uint8_t> tags;
     for (int64_t j = t; j < num_jobs; j += nt) {
       ts_step* st = steps + jobs[j].step_begin;
-      if (!count_widths_job(jobs[j], st, leaves, held, tags)) continue;
+      if (!count_widths_job(jobs[j], st, leaves, tensors, tags)) continue;
       for (int32_t i = 0; i < jobs[j].num_steps; ++i) {
         st[i].pad[0] = tags[i];
         st[i].flags |= TS_STEP_WIDTHS;
