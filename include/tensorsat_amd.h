@@ -233,6 +233,10 @@ int ts_batch_run(const ts_batch* b, ts_stream stream);
  * a product, sum or shift past 2^64 sets overflow[instance] to 1 (the count is then
  * invalid).  mode/early_exit/verdicts are ignored. */
 int ts_batch_count(const ts_batch* b, uint64_t* counts, int32_t* overflow, ts_stream stream);
+/* Writes storage widths (tsc_count_tags: one byte per step, on the device) into the step records
+ * on the device: pad[0] and TS_STEP_WIDTHS where the byte is not 0 (TS_STEP_PACKET and
+ * TS_STEP_PEND are cleared there), no TS_STEP_WIDTHS where it is. */
+int ts_count_tag(ts_step* steps_dev, const uint8_t* tags_dev, int64_t num_steps, ts_stream stream);
 
 /* Keep the entries of order[0..n) whose instance is not yet decided SAT: they are written
  * to out[0..*out_count) (*out_count must be zeroed by the caller; relative order within a

@@ -167,6 +167,10 @@ int tsc_packetize(ts_job* jobs, int64_t num_jobs, ts_step* steps, int64_t num_st
  * as they are: a uint32 tensor fills half its room.  threads <= 0: hardware concurrency. */
 int tsc_count_widths(const ts_job* jobs, int64_t num_jobs, ts_step* steps, int64_t num_steps,
                      const uint8_t* leaves, int64_t num_leaf_bytes, int32_t threads);
+/* The same widths as one byte per step (0: uint64, checked), the records left as they are:
+ * for ts_count_tag, which writes them into a program's device copy. */
+int tsc_count_tags(const ts_job* jobs, int64_t num_jobs, const ts_step* steps, int64_t num_steps,
+                   const uint8_t* leaves, int64_t num_leaf_bytes, uint8_t* tags, int32_t threads);
 
 /* Lane form of a packet-form program (no counterpart in the reference: an execution
  * layout of this build): one 16-byte record per lane of every packet, all index math

@@ -28,6 +28,7 @@
 #include <cstdint>
 #include <cstring>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "tensorsat_prog.h"
@@ -239,7 +240,7 @@ struct JobTensors {
 // leaf entries that no step wrote to): first who reads what, by offset, then whether any write
 // overlaps a tensor that is still to be read.
 bool count_widths_job(const ts_job& job, const ts_step* st, const uint8_t* leaves, JobTensors& T,
-                      std::vector<uint8_t>& tags) {
+                      uint8_t* tags /* per step */) {
   const int n = job.num_steps;
   size_t cap = 64;
   while (cap < 4u * (size_t)(n + 1)) cap *= 2;
@@ -249,10 +250,9 @@ bool count_widths_job(const ts_job& job, const ts_step* st, const uint8_t* leave
   T.reads.assign(2 * (size_t)n, -1);
   T.leaf_off.clear();
   T.leaf_end.clear();
-  tags.assign(n, 0);
-  int leaf_bits = 0;
-  for (int32_t i = 0; i < job.num_leaf_bytes; ++i)
-    if (leaves[job.leaf_begin + i] > 1) leaf_bits = 8;
+  uint8_t all = 0;
+  for (int32_t i = 0; i < job.num_leaf_bytes; ++i) all |= leaves[job.leaf_begin + i];
+  const int leaf_bits = all > 1 ? 8 : 0;
   auto leaf = [&](uint32_t off, int rank) {
     T.leaf_off.push_back((int)off);
     T.leaf_end.push_back((int)(off + (1u << rank)));
@@ -314,44 +314,64 @@ bool count_widths_job(const ts_job& job, const ts_step* st, const uint8_t* leave
 
 }  // namespace
 
-extern "C" int tsc_count_widths(const ts_job* jobs, int64_t num_jobs, ts_step* steps, int64_t num_steps,
-                                const uint8_t* leaves, int64_t num_leaf_bytes, int32_t threads) {
-  if (num_jobs < 0 || num_steps < 0 || num_leaf_bytes < 0 || (num_jobs > 0 && !jobs) || (num_steps > 0 && !steps) ||
-      (num_leaf_bytes > 0 && !leaves))
+// Jobs that share step records must agree on their tags: true if any two do.
+static bool shared_records(const ts_job* jobs, int64_t num_jobs) {
+  std::vector<std::pair<int32_t, int32_t>> r((size_t)num_jobs);
+  for (int64_t j = 0; j < num_jobs; ++j) r[j] = {jobs[j].step_begin, jobs[j].num_steps};
+  auto before = [](const std::pair<int32_t, int32_t>& x, const std::pair<int32_t, int32_t>& y) { return x.first < y.first; };
+  if (!std::is_sorted(r.begin(), r.end(), before)) std::sort(r.begin(), r.end(), before);
+  int64_t end = 0;
+  for (const auto& x : r) {
+    if (x.second > 0 && x.first < end) return true;
+    end = std::max<int64_t>(end, (int64_t)x.first + x.second);
+  }
+  return false;
+}
+
+extern "C" int tsc_count_tags(const ts_job* jobs, int64_t num_jobs, const ts_step* steps, int64_t num_steps,
+                              const uint8_t* leaves, int64_t num_leaf_bytes, uint8_t* tags, int32_t threads) {
+  if (num_jobs < 0 || num_steps < 0 || num_leaf_bytes < 0 || (num_jobs > 0 && !jobs) ||
+      (num_steps > 0 && (!steps || !tags)) || (num_leaf_bytes > 0 && !leaves))
     return TSP_EINVAL;
   for (int64_t j = 0; j < num_jobs; ++j)
     if (jobs[j].step_begin < 0 || jobs[j].num_steps < 0 || (int64_t)jobs[j].step_begin + jobs[j].num_steps > num_steps ||
         jobs[j].leaf_begin < 0 || jobs[j].num_leaf_bytes < 0 ||
         jobs[j].leaf_begin + jobs[j].num_leaf_bytes > num_leaf_bytes)
       return TSP_EINVAL;
-  for (int64_t i = 0; i < num_steps; ++i) {  // leave the packet form: lanes and lane masks
-    if (steps[i].flags & TS_STEP_PACKET) std::memset(&steps[i].o_lpos[16], TS_NOPOS, 8);
-    steps[i].pad[0] = 0;
-    steps[i].flags &= (uint8_t)~(TS_STEP_WIDTHS | TS_STEP_PACKET | TS_STEP_PEND);
-  }
-  // Jobs that share step records must agree on their tags: such programs stay uint64.
-  std::vector<uint8_t> used((size_t)num_steps, 0);
-  for (int64_t j = 0; j < num_jobs; ++j)
-    for (int32_t i = 0; i < jobs[j].num_steps; ++i)
-      if (used[jobs[j].step_begin + i]++) return TSP_OK;
+  if (num_steps > 0) std::memset(tags, 0, (size_t)num_steps);
+  if (shared_records(jobs, num_jobs)) return TSP_OK;
   int nt = threads > 0 ? threads : (int)std::max(1u, std::thread::hardware_concurrency());
   nt = (int)std::max<int64_t>(1, std::min<int64_t>(nt, num_jobs / 64 + 1));
   auto work = [&](int t) {
     JobTensors tensors;
-    std::vector<uint8_t> tags;
     for (int64_t j = t; j < num_jobs; j += nt) {
-      ts_step* st = steps + jobs[j].step_begin;
-      if (!count_widths_job(jobs[j], st, leaves, tensors, tags)) continue;
-      for (int32_t i = 0; i < jobs[j].num_steps; ++i) {
-        st[i].pad[0] = tags[i];
-        st[i].flags |= TS_STEP_WIDTHS;
-      }
+      uint8_t* own = tags + jobs[j].step_begin;
+      if (!count_widths_job(jobs[j], steps + jobs[j].step_begin, leaves, tensors, own) && jobs[j].num_steps > 0)
+        std::memset(own, 0, (size_t)jobs[j].num_steps);
     }
   };
   std::vector<std::thread> pool;
   for (int t = 1; t < nt; ++t) pool.emplace_back(work, t);
   work(0);
   for (auto& th : pool) th.join();
+  return TSP_OK;
+}
+
+extern "C" int tsc_count_widths(const ts_job* jobs, int64_t num_jobs, ts_step* steps, int64_t num_steps,
+                                const uint8_t* leaves, int64_t num_leaf_bytes, int32_t threads) {
+  std::vector<uint8_t> tags((size_t)std::max<int64_t>(num_steps, 0));
+  const int rc = tsc_count_tags(jobs, num_jobs, steps, num_steps, leaves, num_leaf_bytes, tags.data(), threads);
+  if (rc != TSP_OK) return rc;
+  for (int64_t i = 0; i < num_steps; ++i) {
+    if (steps[i].flags & TS_STEP_PACKET) std::memset(&steps[i].o_lpos[16], TS_NOPOS, 8);  // leave the packet form
+    steps[i].flags &= (uint8_t)~(TS_STEP_WIDTHS | TS_STEP_PACKET | TS_STEP_PEND);
+    steps[i].pad[0] = tags[i];
+  }
+  for (int64_t j = 0; j < num_jobs; ++j) {  // a tagged job's first step reads leaves: its tag is not 0
+    ts_step* st = steps + jobs[j].step_begin;
+    if (jobs[j].num_steps > 0 && st[0].pad[0])
+      for (int32_t i = 0; i < jobs[j].num_steps; ++i) st[i].flags |= TS_STEP_WIDTHS;
+  }
   return TSP_OK;
 }
 

@@ -430,16 +430,21 @@ class BatchCounter:
     """
     Exact model counts of all jobs of a program in one persistent launch
     (``ts_batch_count``): tensors stored as uint32 where their entries provably fit and as
-    uint64 elsewhere (:func:`program.count_widths`), per-instance sums of result x 2^free_vars,
+    uint64 elsewhere (:func:`program.count_tags`), per-instance sums of result x 2^free_vars,
     overflow flags raised instead of wrapping.
     """
 
     def __init__(self, prog: Program, *, num_workgroups: int | None = None, device: str = "cuda") -> None:
         torch = _torch()
         L = N.lib()
-        self.dp = DeviceProgram(PG.count_widths(prog), device)
+        self.dp = DeviceProgram(prog, device)
         self.prog = prog
         nj = len(prog.jobs)
+        if len(prog.steps):  # storage widths into the device records, complete for every stream
+            tags = torch.from_numpy(PG.count_tags(prog)).to(device)
+            N.check(L.ts_count_tag(N.dptr(self.dp.steps), N.dptr(tags), len(prog.steps), N.stream_ptr()),
+                    "ts_count_tag")
+            torch.cuda.current_stream().synchronize()
         if num_workgroups is None:
             mx = N.i32(0)
             N.check(L.ts_batch_max_workgroups(ctypes.byref(mx)), "ts_batch_max_workgroups")

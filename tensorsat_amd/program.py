@@ -96,6 +96,8 @@ def _lib():
         L.tsc_lanes.argtypes = [vp, ctypes.c_int64, vp, ctypes.c_int64, vp, ctypes.c_int64, vp, ctypes.c_int32]
         L.tsc_count_widths.argtypes = [vp, ctypes.c_int64, vp, ctypes.c_int64, vp, ctypes.c_int64, ctypes.c_int32]
         L.tsc_count_widths.restype = ctypes.c_int
+        L.tsc_count_tags.argtypes = [vp, ctypes.c_int64, vp, ctypes.c_int64, vp, ctypes.c_int64, vp, ctypes.c_int32]
+        L.tsc_count_tags.restype = ctypes.c_int
         for f in (L.tsc_compile, L.tsc_sat_batch, L.tsc_program_sizes, L.tsc_program_copy, L.tsp_elim,
                   L.tsp_elim_order, L.tsp_order_cost, L.tsp_elim_order_prior, L.tsc_packetize, L.tsc_lanes):
             f.restype = ctypes.c_int
@@ -424,6 +426,17 @@ def count_widths(prog: Program, threads: int = 0) -> Program:
                                          leaves.ctypes.data, leaves.size, int(threads)), "tsc_count_widths")
     meta = {k: v for k, v in prog.meta.items() if k != "packetized"}
     return Program(prog.jobs, steps, prog.leaves, prog.stats, meta)
+
+
+def count_tags(prog: Program, threads: int = 0) -> np.ndarray:
+    """The storage widths of :func:`count_widths` as one byte per step (``tsc_count_tags``; 0:
+    uint64), for the device copy of ``prog``'s records."""
+    tags = np.empty(len(prog.steps), np.uint8)
+    steps = np.ascontiguousarray(prog.steps)
+    leaves = np.ascontiguousarray(prog.leaves, dtype=np.uint8)
+    _plan._check(_lib().tsc_count_tags(prog.jobs.ctypes.data, len(prog.jobs), steps.ctypes.data, len(steps),
+                                       leaves.ctypes.data, leaves.size, tags.ctypes.data, int(threads)), "tsc_count_tags")
+    return tags
 
 
 LANE_DTYPE = np.dtype(

@@ -191,3 +191,34 @@ def test_records_without_widths_count_as_uint64():
             counter = BatchCounter(other)
             counter.dp = DeviceProgram(other)  # the records as they are
             assert counter.run() == want
+
+
+def test_tags_are_the_widths():
+    for prog in (*_packet_programs(), _disjoint(23), *(_steps_by_hand(k)[0] for k in ("upper half", "whole"))):
+        for form in (prog, PG.packetize(prog)) if int(prog.steps["out_rank"].max()) <= 6 else (prog,):
+            before = form.steps.copy()
+            tags = PG.count_tags(form)
+            assert (form.steps == before).all()
+            np.testing.assert_array_equal(tags, PG.count_widths(form).steps["pad"][:, 0])
+
+
+@pytest.mark.gpu
+def test_device_records_carry_the_widths():
+    """The records of a counter on the device are count_widths' (lane masks apart), whatever
+    form or widths they had before."""
+    from tensorsat_amd.executor import BatchCounter
+
+    for prog in (*_packet_programs(), _disjoint(23), _steps_by_hand("upper half")[0]):
+        stale = PG.count_widths(prog)
+        forms = [prog, stale]
+        if int(prog.steps["out_rank"].max()) <= 6:
+            forms.append(PG.packetize(prog))
+        for form in forms:
+            got = BatchCounter(form).dp.steps.cpu().numpy().view(PG.STEP_DTYPE)
+            want = PG.count_widths(form).steps
+            tagged = want["pad"][:, 0] != 0
+            np.testing.assert_array_equal(got["pad"][tagged], want["pad"][tagged])
+            np.testing.assert_array_equal(got["flags"][tagged], want["flags"][tagged])
+            assert not (got["flags"][~tagged] & PG.STEP_WIDTHS).any()
+            for name in ("lhs_off", "rhs_off", "out_off", "out_rank", "sum_rank", "c_lpos", "o_rpos"):
+                np.testing.assert_array_equal(got[name], want[name])
