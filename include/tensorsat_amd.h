@@ -226,13 +226,16 @@ typedef struct {
  * workgroup, OR-ing the scalar result into verdicts[instance]. */
 int ts_batch_run(const ts_batch* b, ts_stream stream);
 
-/* Counting variant (#SAT): arenas have room for uint64 entries (arena_stride in bytes, >= 8 x
- * the largest arena_elems); tensors are uint64 unless a step's TS_STEP_WIDTHS flag and pad[0]
- * say uint32 (tsc_count_widths), and records in packet form count as any others.  Every
- * job's scalar result times 2^free_vars is added to counts[instance] (zeroed by the caller);
- * a product, sum or shift past 2^64 sets overflow[instance] to 1 (the count is then
- * invalid).  mode/early_exit/verdicts are ignored. */
+/* Counting variant (#SAT): arenas hold uint64 entries (arena_stride in bytes, >= 8 x the
+ * largest arena_elems), every job's scalar result times 2^free_vars is added to
+ * counts[instance] (zeroed by the caller); a product, sum or shift past 2^64 sets
+ * overflow[instance] to 1 (the count is then invalid).  mode/early_exit/verdicts and the
+ * records' pad are ignored. */
 int ts_batch_count(const ts_batch* b, uint64_t* counts, int32_t* overflow, ts_stream stream);
+/* The same counts with tensors stored as uint32 where a step's TS_STEP_WIDTHS flag and pad[0]
+ * say so (tsc_count_widths, ts_count_tag; arenas as above); other steps run on uint64, and
+ * programs without any widths faster by ts_batch_count. */
+int ts_batch_count_widths(const ts_batch* b, uint64_t* counts, int32_t* overflow, ts_stream stream);
 /* Writes storage widths (tsc_count_tags: one byte per step, on the device) into the step records
  * on the device: pad[0] and TS_STEP_WIDTHS where the byte is not 0 (TS_STEP_PACKET and
  * TS_STEP_PEND are cleared there), no TS_STEP_WIDTHS where it is. */

@@ -47,8 +47,9 @@ typedef struct {
 #define TS_STEP_PEND 8    /* packet form: last record of its packet */
 #define TS_STEP_WIDTHS 16 /* counting (tsc_count_widths): pad[0] = storage widths, TS_COUNT_* */
 /* pad[0] of a TS_STEP_WIDTHS step holds the storage of its operands (bits 0-1 lhs, 2-3 rhs: 0
- * uint64, 1 uint32, 2 uint64 with values below 2^32) and these bits.  Steps without the flag
- * are counted in uint64 throughout, checked, whatever pad holds.  A step has this flag or
+ * uint64, 1 uint32, 2 uint64 with values below 2^32) and these bits, for
+ * ts_batch_count_widths.  Steps without the flag, and all steps of ts_batch_count, are counted
+ * in uint64 throughout, checked, whatever pad holds.  A step has this flag or
  * TS_STEP_PACKET, never both: each gives pad[0] its meaning. */
 #define TS_COUNT_OUT32 16 /* the result is stored as uint32 */
 #define TS_COUNT_EXACT 32 /* no product or sum of this step reaches 2^64 */

@@ -41,7 +41,7 @@ EXPORTS = (
     "ts_init", "ts_version", "ts_contract2", "ts_contract2_scratch", "ts_contract2_into", "ts_rewire", "ts_spider", "ts_union", "ts_stack",
     "ts_select", "ts_as_scalar", "ts_diagonal", "ts_count_contract2", "ts_bytes_to_u64",
     "ts_program_run", "ts_program_count", "ts_batch_run", "ts_batch_max_workgroups",
-    "ts_batch_compact", "ts_batch_count", "ts_count_tag", "ts_batch_max_workgroups_lds", "ts_gnn_gemm", "ts_gnn_wgrad", "ts_gnn_wgrad_scratch",
+    "ts_batch_compact", "ts_batch_count", "ts_batch_count_widths", "ts_count_tag", "ts_batch_max_workgroups_lds", "ts_gnn_gemm", "ts_gnn_wgrad", "ts_gnn_wgrad_scratch",
     "ts_gnn_segsum", "ts_gnn_relu_back",
     "ts_gnn_head", "ts_gnn_adam", "ts_gnn_cast_bf16", "ts_dense_config", "ts_dense_tiles", "ts_dense_tile_of",
     "ts_search_run", "ts_search_run_queue", "ts_search_decide_noalloc", "ts_program_run_fused", "ts_program_run_gang",
@@ -98,6 +98,7 @@ def load() -> ctypes.CDLL:
         L.ts_count_tag.argtypes = [vp, vp, i64, vp]
         L.ts_batch_compact.argtypes = [vp, i32, vp, vp, vp, vp, vp]
         L.ts_batch_count.argtypes = [P(Batch), vp, vp, vp]
+        L.ts_batch_count_widths.argtypes = [P(Batch), vp, vp, vp]
         i8 = ctypes.c_int64
         f32 = ctypes.c_float
         L.ts_gnn_gemm.argtypes = [vp, i8, i8, vp, i8, i8, vp, i8, i32, i32, i32, vp, i32, i32, i32, vp]

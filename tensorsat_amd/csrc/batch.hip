@@ -473,15 +473,18 @@ __global__ __launch_bounds__(64) void k_batch_wave(ts_batch b) {
 
 // ---- counting semiring ---------------------------------------------------------------
 //
-// The same walk over (+, x) with exact integer counts: an arena element is 8 bytes wide, and
-// a tensor whose record proves its entries below 2^32 (tsc_count_widths: at most 2^b with b
-// the summed bits under it) is stored as uint32 at the start of its room, so a step reads and
-// writes half the bytes.  Records without that proof (no TS_STEP_WIDTHS) are uint64 with
-// checked arithmetic.  Bound by memory traffic: a width-18 job's arena is 1.3 MB and 1536 of them are
-// in flight, far beyond the caches.  n=100, m=300 over 46816 cubes of width 18 (23 G elements
-// read and written): 84 ms with uint64 tensors and one thread per output, 66 ms with uint32
-// ones (the longest sums of 2^16 terms on one thread then hold their job for 40 ms), 51 ms
-// with long sums shared out over a wave and the jobs taken longest first.
+// The same walk over (+, x) with exact integer counts, in two kernels.  k_batch_count<false>:
+// uint64 entries, checked arithmetic, one output per thread (step_u64).  k_batch_count<true>: an
+// arena element is 8 bytes wide, and a tensor whose record proves its entries below 2^32
+// (tsc_count_widths: at most 2^b with b the summed bits under it) is stored as uint32 at the
+// start of its room, so a step reads and writes half the bytes; records without that proof (no
+// TS_STEP_WIDTHS) are uint64 with checked arithmetic.  Bound by memory traffic: a width-18
+// job's arena is 1.3 MB and 1536 of them are in flight, far beyond the caches.  n=100, m=300
+// over 46816 cubes of width 18 (23 G elements read and written): 84 ms by the first kernel, 66
+// ms with uint32 tensors (the longest sums of 2^16 terms on one thread then hold their job for
+// 40 ms), 51 ms with long sums shared out over a wave and the jobs taken longest first.  Small
+// tensors stay in the caches, where the first kernel is ahead: 20 variables at width 9 62 and
+// 78 us, 40 at width 12 129 and 121.
 struct CountTag {
   uint32_t v;
   __device__ uint32_t lhs() const { return v & 3u; }          // 0 uint64, 1 uint32, 2 uint64 below 2^32
@@ -698,6 +701,7 @@ __global__ __launch_bounds__(256) void k_count_tag(uint32_t* __restrict__ steps,
   }
 }
 
+template <bool WIDTHS>
 __global__ __launch_bounds__(CWG) void k_batch_count(ts_batch b, unsigned long long* __restrict__ counts,
                                                     int32_t* __restrict__ overflow) {
   __shared__ Lut L;
@@ -730,9 +734,17 @@ __global__ __launch_bounds__(CWG) void k_batch_count(ts_batch b, unsigned long l
       __syncthreads();
       for (int s = 0; s < ns; ++s) {
         const ts_step& st = s_steps[s];
-        // flags and pad[0] in one read.  Without widths (in packet form pad[0] is a lane) the step
-        // is a general one on uint64 tensors; the tag itself stays as read, a select on it cost
-        // every step 2 % (n=60, width 17: 1445 us, 1426 so).
+        if constexpr (!WIDTHS) {  // uint64 throughout, pad ignored
+          build_lut(st, L, !(st.flags & TS_STEP_KINNER) && st.sum_rank > 0, tid);
+          __syncthreads();
+          const uint64_t* rhs = arena + ((st.flags & TS_STEP_NORHS) ? st.lhs_off : st.rhs_off);
+          ovf |= step_u64(st, L, arena + st.lhs_off, rhs, arena + st.out_off, (uint64_t)tid, (uint64_t)CWG);
+          __syncthreads();
+          continue;
+        }
+        // flags and pad[0] in one read.  A step without widths is a general one on uint64
+        // tensors; the tag itself stays as read, a select on it cost every step 2 % (n=60, width
+        // 17: 1445 us, 1426 so).
         const uint32_t fl = *reinterpret_cast<const uint32_t*>(&st.flags);
         const CountTag tag{(fl >> 8) & 255u};
         const bool kinner = fl & TS_STEP_KINNER, norhs = fl & TS_STEP_NORHS, widths = fl & TS_STEP_WIDTHS;
@@ -821,6 +833,18 @@ __global__ __launch_bounds__(WG) void k_compact(const int32_t* __restrict__ orde
   }
 }
 
+template <bool WIDTHS>
+int launch_count(const ts_batch* b, uint64_t* counts, int32_t* overflow, ts_stream stream) {
+  if (!b || !counts || !overflow || b->num_jobs < 0 || b->num_workgroups <= 0 || !b->counter) return TS_EINVAL;
+  if (b->num_workgroups < QSEG && b->num_jobs > 2 * (int64_t)b->num_workgroups) return TS_EINVAL;
+  if (b->num_jobs > 0 && (!b->jobs || !b->steps || !b->leaves || !b->arenas)) return TS_EINVAL;
+  if (b->arena_stride <= 0 || (b->arena_stride & 255)) return TS_EINVAL;
+  if (b->num_jobs == 0) return TS_OK;
+  hipLaunchKernelGGL((k_batch_count<WIDTHS>), dim3(b->num_workgroups), dim3(CWG), 0,
+                     reinterpret_cast<hipStream_t>(stream), *b, reinterpret_cast<unsigned long long*>(counts), overflow);
+  return hipGetLastError() == hipSuccess ? TS_OK : TS_EHIP;
+}
+
 }  // namespace
 
 extern "C" {
@@ -886,14 +910,11 @@ int ts_batch_run(const ts_batch* b, ts_stream stream) {
 }
 
 int ts_batch_count(const ts_batch* b, uint64_t* counts, int32_t* overflow, ts_stream stream) {
-  if (!b || !counts || !overflow || b->num_jobs < 0 || b->num_workgroups <= 0 || !b->counter) return TS_EINVAL;
-  if (b->num_workgroups < QSEG && b->num_jobs > 2 * (int64_t)b->num_workgroups) return TS_EINVAL;
-  if (b->num_jobs > 0 && (!b->jobs || !b->steps || !b->leaves || !b->arenas)) return TS_EINVAL;
-  if (b->arena_stride <= 0 || (b->arena_stride & 255)) return TS_EINVAL;
-  if (b->num_jobs == 0) return TS_OK;
-  hipLaunchKernelGGL(k_batch_count, dim3(b->num_workgroups), dim3(CWG), 0, reinterpret_cast<hipStream_t>(stream),
-                     *b, reinterpret_cast<unsigned long long*>(counts), overflow);
-  return hipGetLastError() == hipSuccess ? TS_OK : TS_EHIP;
+  return launch_count<false>(b, counts, overflow, stream);
+}
+
+int ts_batch_count_widths(const ts_batch* b, uint64_t* counts, int32_t* overflow, ts_stream stream) {
+  return launch_count<true>(b, counts, overflow, stream);
 }
 
 int ts_count_tag(ts_step* steps_dev, const uint8_t* tags_dev, int64_t num_steps, ts_stream stream) {

@@ -429,19 +429,30 @@ class BatchExecutor:
 class BatchCounter:
     """
     Exact model counts of all jobs of a program in one persistent launch
-    (``ts_batch_count``): tensors stored as uint32 where their entries provably fit and as
-    uint64 elsewhere (:func:`program.count_tags`), per-instance sums of result x 2^free_vars,
+    (``ts_batch_count``, with large tensors ``ts_batch_count_widths``: stored as uint32 where their
+    entries provably fit, :func:`program.count_tags`), per-instance sums of result x 2^free_vars,
     overflow flags raised instead of wrapping.
     """
 
-    def __init__(self, prog: Program, *, num_workgroups: int | None = None, device: str = "cuda") -> None:
+    # Largest tensor's rank from which widths are used.  Below it tensors stay in the caches and
+    # the plain kernel's shorter code wins: 20 variables at width 9 62 us, 78 with widths; 40 at
+    # width 12 129 and 121; 60 at width 14 338 and 227; 60 at width 17 2.31 and 1.42 ms.
+    WIDTHS_RANK = 12
+
+    def __init__(self, prog: Program, *, num_workgroups: int | None = None, device: str = "cuda",
+                 widths: bool | None = None) -> None:
+        """``widths``: use storage widths (default: from tensors of rank ``WIDTHS_RANK`` on)."""
         torch = _torch()
         L = N.lib()
         self.dp = DeviceProgram(prog, device)
         self.prog = prog
         nj = len(prog.jobs)
-        if len(prog.steps):  # storage widths into the device records, complete for every stream
-            tags = torch.from_numpy(PG.count_tags(prog)).to(device)
+        if widths is None:
+            widths = len(prog.steps) > 0 and int(prog.steps["out_rank"].max()) >= self.WIDTHS_RANK
+        tags = PG.count_tags(prog) if widths else np.zeros(0, np.uint8)
+        self.widths = bool(tags.any())
+        if self.widths:  # into the device records, complete for every stream
+            tags = torch.from_numpy(tags).to(device)
             N.check(L.ts_count_tag(N.dptr(self.dp.steps), N.dptr(tags), len(prog.steps), N.stream_ptr()),
                     "ts_count_tag")
             torch.cuda.current_stream().synchronize()
@@ -478,8 +489,8 @@ class BatchCounter:
             verdicts=self.dummy.data_ptr(), counter=self.counter.data_ptr(), early_exit=0,
             job_done=None, num_jobs_dev=None,
         )
-        N.check(L.ts_batch_count(ctypes.byref(b), N.dptr(self.counts), N.dptr(self.overflow), N.stream_ptr()),
-                "ts_batch_count")
+        count = L.ts_batch_count_widths if self.widths else L.ts_batch_count
+        N.check(count(ctypes.byref(b), N.dptr(self.counts), N.dptr(self.overflow), N.stream_ptr()), "ts_batch_count")
         if events is not None:
             events[1].record()
 

@@ -153,7 +153,8 @@ def test_counts_over_parts_of_tensors(kind):
     from tensorsat_amd.executor import BatchCounter
 
     prog, want = _steps_by_hand(kind)
-    assert BatchCounter(prog).run() == [want]
+    for widths in (True, False, None):
+        assert BatchCounter(prog, widths=widths).run() == [want]
 
 
 def _packet_programs():
@@ -180,7 +181,7 @@ def test_widths_and_lanes_exclude_each_other():
 @pytest.mark.gpu
 def test_records_without_widths_count_as_uint64():
     """Packet-form records (pad[0] = a lane) and records whose pad was never cleared, through
-    the C entry."""
+    both C entries."""
     from tensorsat_amd.executor import BatchCounter, DeviceProgram
 
     for prog in _packet_programs():
@@ -188,9 +189,10 @@ def test_records_without_widths_count_as_uint64():
         dirty = PG.Program(prog.jobs, prog.steps.copy(), prog.leaves, prog.stats, {})
         dirty.steps["pad"] = np.random.default_rng(0).integers(0, 256, dirty.steps["pad"].shape)
         for other in (PG.packetize(prog), dirty):
-            counter = BatchCounter(other)
+            counter = BatchCounter(other, widths=True)
             counter.dp = DeviceProgram(other)  # the records as they are
-            assert counter.run() == want
+            for counter.widths in (True, False):  # ts_batch_count_widths, ts_batch_count
+                assert counter.run() == want
 
 
 def test_tags_are_the_widths():
@@ -214,11 +216,43 @@ def test_device_records_carry_the_widths():
         if int(prog.steps["out_rank"].max()) <= 6:
             forms.append(PG.packetize(prog))
         for form in forms:
-            got = BatchCounter(form).dp.steps.cpu().numpy().view(PG.STEP_DTYPE)
+            got = BatchCounter(form, widths=True).dp.steps.cpu().numpy().view(PG.STEP_DTYPE)
             want = PG.count_widths(form).steps
             tagged = want["pad"][:, 0] != 0
+            if not tagged.any():  # counted by ts_batch_count, which ignores them
+                continue
             np.testing.assert_array_equal(got["pad"][tagged], want["pad"][tagged])
             np.testing.assert_array_equal(got["flags"][tagged], want["flags"][tagged])
             assert not (got["flags"][~tagged] & PG.STEP_WIDTHS).any()
             for name in ("lhs_off", "rhs_off", "out_off", "out_rank", "sum_rank", "c_lpos", "o_rpos"):
                 np.testing.assert_array_equal(got[name], want[name])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("widths", [True, False])
+def test_both_kernels_count_alike(widths):
+    """Edges of uint32 and uint64, brute force, wide and general steps, by either kernel."""
+    from tensorsat_amd.executor import BatchCounter
+    from wide_steps import wide_sum_program
+
+    for m in (1, 9, 10, 11, 20, 21, 22):
+        assert BatchCounter(_disjoint(m), widths=widths).run() == [7**m], m
+    with pytest.raises(OverflowError):
+        BatchCounter(_disjoint(23), widths=widths).run()
+    for n, width in ((14, 3), (20, 9), (22, 12), (24, 16)):
+        cnfs = [CNFInstance.random(3, n, int(r * n), rng=40 * n + i) for i, r in enumerate((1.0, 2.0, 3.0))]
+        counter = BatchCounter(PG.sat_batch(cnfs, width=width), widths=widths)
+        assert counter.widths is widths
+        assert counter.run() == [brute.count(c.num_vars, c.clauses) for c in cnfs]
+    for permute in (True, False):
+        prog, _ = wide_sum_program(3, out_wires=(), n=10, density=0.5, permute=permute)
+        assert BatchCounter(prog, widths=widths).run() == BatchCounter(prog, widths=not widths).run()
+
+
+@pytest.mark.gpu
+def test_widths_come_with_large_tensors():
+    from tensorsat_amd.executor import BatchCounter
+
+    for width in (8, 14):
+        prog = PG.sat_batch([CNFInstance.random(3, 40, 120, rng=5)], width=width, max_cubes=4)
+        assert BatchCounter(prog).widths is (int(prog.steps["out_rank"].max()) >= BatchCounter.WIDTHS_RANK)
